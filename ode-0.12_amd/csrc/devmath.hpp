@@ -6,6 +6,14 @@
 
 namespace odemi {
 
+// p, known to point into global memory.  Pointers handed to a function that
+// is not inlined are generic, and a generic (flat) load counts as an LDS
+// access too: every wait for LDS would also wait for it.
+template <class T>
+__device__ __forceinline__ T *as_global(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)(unsigned long long)p;
+}
+
 __device__ __forceinline__ float3 mk3(float x, float y, float z) { return make_float3(x, y, z); }
 __device__ __forceinline__ float3 xyz(const float4 &a) { return make_float3(a.x, a.y, a.z); }
 __device__ __forceinline__ float4 f4(const float3 &a, float w = 0.f) { return make_float4(a.x, a.y, a.z, w); }

@@ -198,7 +198,7 @@ enum { PH_AABB = 0, PH_BROAD, PH_NARROW, PH_BODIES, PH_ROWS, PH_ORDER, PH_SOR, P
 
 struct ScratchLayout {
   long long aabb, gbig, gidx, glevel, gdb, cells, ecount, pairs, pkeys, pcount, contacts, cons, rows, btmp,
-      order, adjs, adj, island, color, misc, sor, total;
+      order, adjs, adj, island, color, misc, sor, ref, total;
 };
 
 OD_HD inline long long od_align(long long x) { return (x + 255) & ~255LL; }
@@ -276,6 +276,8 @@ OD_HD inline ScratchLayout scratch_layout(int nb, int ng, int nj, int pcap, int 
   L.color = o;    o = od_align(o + 4LL * (ncons + nb));
   L.misc = o;     o = od_align(o + 4LL * 64);
   L.sor = o;      o = od_align(o + sor_bytes(nb, rcap, (int)ncons, true));
+  // the reference order's solve: 4 + 36 + 160 bytes per row, 28 per body
+  L.ref = o;      o = od_align(o + 200LL * rcap + 28LL * nb + 128);
   L.total = o;
   return L;
 }

@@ -38,6 +38,7 @@ struct Shared {
   float fval[8];
   int ccount[MAX_COLORS_LDS + 1];
   int ccur[MAX_COLORS_LDS];
+  int lcount[4];   // rows of a level (ref_levels)
 };
 
 // dynamic LDS pool of the workgroup (size DevBatch::lds_bytes): sort keys,
@@ -763,163 +764,7 @@ __device__ inline Surf host_surface(const ContactIn &ci) {
   return s;
 }
 
-// relax one row: ode/src/quickstep.cpp:484-582 (J and b scaled by ad there).
-// A body's 6 constraint-force floats are at bt[32 b + 9] (per-body scratch).
-__device__ inline void relax_row(Row *rows, int r, float *bt) {
-  Row &R = rows[r];
-  float old = R.lambda;
-  float *f1 = bt + 32 * R.b1 + 9;
-  float s = R.J[0] * f1[0] + R.J[1] * f1[1] + R.J[2] * f1[2] + R.J[3] * f1[3] + R.J[4] * f1[4] + R.J[5] * f1[5];
-  float *f2 = nullptr;
-  if (R.b2 >= 0) {
-    f2 = bt + 32 * R.b2 + 9;
-    s += R.J[6] * f2[0] + R.J[7] * f2[1] + R.J[8] * f2[2] + R.J[9] * f2[3] + R.J[10] * f2[4] + R.J[11] * f2[5];
-  }
-  float delta = R.ad * (R.rhs - old * R.cfm - s);
-  float lo, hi;
-  if (R.findex >= 0) {
-    hi = fabsf(R.hi * rows[R.findex].lambda);
-    lo = -hi;
-  } else {
-    lo = R.lo;
-    hi = R.hi;
-  }
-  float nl = old + delta;
-  if (nl < lo) { delta = lo - old; R.lambda = lo; }
-  else if (nl > hi) { delta = hi - old; R.lambda = hi; }
-  else R.lambda = nl;
-  for (int k = 0; k < 6; k++) f1[k] += delta * R.iMJ[k];
-  if (f2)
-    for (int k = 0; k < 6; k++) f2[k] += delta * R.iMJ[6 + k];
-}
-
-// LDS bytes of the reference-order solve of a world: its rows, the row
-// order and 6 fc floats per body
-__device__ inline long long ref_sor_lds_bytes(int nrows, int nb) {
-  return (long long)sizeof(Row) * nrows + 8LL * nrows + 24LL * nb;
-}
-// the same with the rows left in global memory: impulses, order and fc only
-__device__ inline long long ref_sor_lds_bytes_streamed(int nrows, int nb) {
-  return 8LL * nrows + 24LL * nb;
-}
-
-// the read-only part of a row (everything but lambda), held in registers
-struct RowC {
-  float J[12], iMJ[12];
-  float rhs, cfm, lo, hi, ad;
-  int findex, b1, b2;
-};
-
-__device__ inline RowC load_rowc(const Row &R) {
-  RowC q;
-  for (int k = 0; k < 12; k++) { q.J[k] = R.J[k]; q.iMJ[k] = R.iMJ[k]; }
-  q.rhs = R.rhs; q.cfm = R.cfm; q.lo = R.lo; q.hi = R.hi; q.ad = R.ad;
-  q.findex = R.findex; q.b1 = R.b1; q.b2 = R.b2;
-  return q;
-}
-
-// relax_row on a row held in registers, its impulse in lam[r] and fc in
-// F[6 b]: the same arithmetic in the same order.  All reads (the row's
-// impulse, its normal row's impulse, both bodies' fc) are issued before any
-// write, so they share one LDS round trip.
-__device__ inline void relax_rowc(const RowC &R, int r, float *lam, float *F) {
-  const bool two = R.b2 >= 0;
-  const float old = lam[r];
-  const float lf = lam[R.findex >= 0 ? R.findex : r];
-  float *f1 = F + 6 * R.b1;
-  float *f2 = F + 6 * (two ? R.b2 : R.b1);
-  float fa[6], fb[6];
-  for (int k = 0; k < 6; k++) { fa[k] = f1[k]; fb[k] = f2[k]; }
-  float s = R.J[0] * fa[0] + R.J[1] * fa[1] + R.J[2] * fa[2] + R.J[3] * fa[3] + R.J[4] * fa[4] + R.J[5] * fa[5];
-  if (two) s += R.J[6] * fb[0] + R.J[7] * fb[1] + R.J[8] * fb[2] + R.J[9] * fb[3] + R.J[10] * fb[4] + R.J[11] * fb[5];
-  float delta = R.ad * (R.rhs - old * R.cfm - s);
-  float lo, hi;
-  if (R.findex >= 0) {
-    hi = fabsf(R.hi * lf);
-    lo = -hi;
-  } else {
-    lo = R.lo;
-    hi = R.hi;
-  }
-  float nl = old + delta;
-  if (nl < lo) { delta = lo - old; lam[r] = lo; }
-  else if (nl > hi) { delta = hi - old; lam[r] = hi; }
-  else lam[r] = nl;
-  for (int k = 0; k < 6; k++) f1[k] = fa[k] + delta * R.iMJ[k];
-  if (two)
-    for (int k = 0; k < 6; k++) f2[k] = fb[k] + delta * R.iMJ[6 + k];
-}
-
-// SOR_LCP in the reference order (quickstep.cpp:406-582): one island per
-// lane; rows ordered with the findex = -1 rows first and the others from the
-// tail, reshuffled every 8 iterations with the island's own RNG state.
-// MODE 1: rows, impulses, order and fc in the LDS pool (copied in first and
-// back after the iterations); MODE 2 (worlds whose rows exceed the pool):
-// impulses, order and fc in LDS, the read-only rows streamed from global
-// memory; in both the next row's read-only part is loaded while the current
-// one is relaxed.  MODE 0: everything in the world's scratch (rows, ord, and
-// fc at bt[32 b + 9]).  The arithmetic and its order are the same in all
-// three.
-template <int MODE>
-__device__ void sor_reference(Row *rows, float *bt, const int *isl, int *ord, int nrows, int ngroups, int nb,
-                              int iters) {
-  constexpr bool LDS = MODE == 1;
-  Row *R = LDS ? (Row *)od_pool : rows;
-  int *O = LDS ? (int *)(R + nrows) : (MODE == 2 ? (int *)od_pool : ord);
-  float *F = MODE == 0 ? bt : (float *)(O + nrows);
-  float *LAM = MODE == 0 ? nullptr : F + 6 * nb;
-  const int nt = blockDim.x;
-  if (MODE != 0) {
-    if (LDS)
-      for (int i = threadIdx.x; i < nrows; i += nt) R[i] = rows[i];
-    for (int i = threadIdx.x; i < nrows; i += nt) LAM[i] = rows[i].lambda;
-    for (int b = threadIdx.x; b < nb; b += nt)
-      for (int k = 0; k < 6; k++) F[6 * b + k] = bt[32 * b + 9 + k];
-    __syncthreads();
-  }
-  for (int k = threadIdx.x; k < ngroups; k += nt) {
-    int r0 = isl[5 * k + 2], m = isl[5 * k + 3];
-    if (m <= 0) continue;
-    unsigned seed = (unsigned)isl[5 * k + 4];
-    int *o = O + r0;
-    int head = 0, tail = m - 1;
-    for (int i = 0; i < m; i++) {
-      if (R[r0 + i].findex == -1) o[head++] = r0 + i;
-      else o[tail--] = r0 + i;
-    }
-    for (int it = 0; it < iters; it++) {
-      if ((it & 7) == 0) {
-        for (int i = 1; i < m; i++) {
-          int sw = lcg_below(seed, i + 1);
-          int t = o[i]; o[i] = o[sw]; o[sw] = t;
-        }
-      }
-      if (MODE != 0) {
-        // two row buffers in turn: the next row loads while this one relaxes
-        int ra = o[0], rb = ra;
-        RowC qa = load_rowc(R[ra]), qb;
-        for (int i = 0; i < m; i += 2) {
-          if (i + 1 < m) { rb = o[i + 1]; qb = load_rowc(R[rb]); }
-          relax_rowc(qa, ra, LAM, F);
-          if (i + 1 >= m) break;
-          if (i + 2 < m) { ra = o[i + 2]; qa = load_rowc(R[ra]); }
-          relax_rowc(qb, rb, LAM, F);
-        }
-      } else {
-        for (int i = 0; i < m; i++) relax_row(R, o[i], F);
-      }
-    }
-  }
-  // islands are solved by lanes of every wavefront; the integration reads
-  // the fc of all bodies
-  __syncthreads();
-  if (MODE != 0) {
-    for (int i = threadIdx.x; i < nrows; i += nt) rows[i].lambda = LAM[i];
-    for (int b = threadIdx.x; b < nb; b += nt)
-      for (int k = 0; k < 6; k++) bt[32 * b + 9 + k] = F[6 * b + k];
-    __syncthreads();
-  }
-}
+#include "ref_solver.hpp"
 
 // |lambda - clamp(lambda - d, lo, hi)| evaluated without the cancellation of
 // lambda - (lambda - d): |d| when the step stays inside the bounds, else the
@@ -2138,15 +1983,19 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
   // --- SOR-LCP
   const int iters = P.iterations;
   if (ref) {
-    int *ord = corder + ncons + nb;
+    // the placement with as much as fits in the LDS pool
+    char *gws = c.at<char>(c.L.ref);
+    const long long st = ref_state_bytes(nrows, nb), sched = ref_sched_bytes(nrows, nb);
     if (P.exact && B.lcp_ws)
       lcp_exact_world(B, c.w, rows, bt, isl, ngroups, nb, sh);
-    else if (ref_sor_lds_bytes(nrows, nb) <= B.lds_bytes)
-      sor_reference<1>(rows, bt, isl, ord, nrows, ngroups, nb, iters);
-    else if (ref_sor_lds_bytes_streamed(nrows, nb) <= B.lds_bytes)
-      sor_reference<2>(rows, bt, isl, ord, nrows, ngroups, nb, iters);
+    else if (st + sched + ref_sides_bytes(nrows) <= B.lds_bytes)
+      sor_reference<REF_IN_LDS>(rows, bt, isl, gws, (LdsChar *)od_pool, nrows, ngroups, nb, iters, sh);
+    else if (st + sched <= B.lds_bytes)
+      sor_reference<REF_ROWS_GLOBAL>(rows, bt, isl, gws, (LdsChar *)od_pool, nrows, ngroups, nb, iters, sh);
+    else if (st <= B.lds_bytes)
+      sor_reference<REF_SCHED_GLOBAL>(rows, bt, isl, gws, (LdsChar *)od_pool, nrows, ngroups, nb, iters, sh);
     else
-      sor_reference<0>(rows, bt, isl, ord, nrows, ngroups, nb, iters);
+      sor_reference<REF_IN_GLOBAL>(rows, bt, isl, gws, (LdsChar *)od_pool, nrows, ngroups, nb, iters, sh);
     if (threadIdx.x == 0) B.counters[c.w * CNT_N + CNT_ITERS] = iters;
   } else if (STAGE == 1) {
     // the sweeps run in their own kernel
