@@ -14,6 +14,28 @@ __device__ __forceinline__ T *as_global(T *p) {
   return (T *)(__attribute__((address_space(1))) T *)(unsigned long long)p;
 }
 
+// A value that is the same in every lane, kept as such: the arguments of a
+// function that is not inlined arrive per lane, and branches and addresses
+// made from them would be worked out per lane too.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ bool uniform(bool v) { return __builtin_amdgcn_readfirstlane(v ? 1 : 0) != 0; }
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+template <class T>
+__device__ __forceinline__ T *uniform_global(T *p) {
+  const unsigned long long a = (unsigned long long)p;
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32));
+  return as_global((T *)(((unsigned long long)hi << 32) | lo));
+}
+// a byte of the workgroup's LDS, and its uniform address
+typedef __attribute__((address_space(3))) char LdsChar;
+typedef __attribute__((address_space(3))) float LdsFloat;
+__device__ __forceinline__ LdsChar *uniform(LdsChar *p) {
+  return (LdsChar *)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned long long)p);
+}
+
 __device__ __forceinline__ float3 mk3(float x, float y, float z) { return make_float3(x, y, z); }
 __device__ __forceinline__ float3 xyz(const float4 &a) { return make_float3(a.x, a.y, a.z); }
 __device__ __forceinline__ float4 f4(const float3 &a, float w = 0.f) { return make_float4(a.x, a.y, a.z, w); }

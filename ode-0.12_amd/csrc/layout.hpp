@@ -158,31 +158,16 @@ struct Cons {
   int fb;                  // feedback slot or -1
 };
 
-// Compact SOR row (64 bytes) used by the coloured solver.  J_l2 = -J_l1
-// for every row the supported joints produce, and inv(M) J^T is recomputed
-// from the per-body inverse mass and world inverse inertia, so a row needs
-// only J_l1, J_a1, J_a2 and its scalars.
+// SOR row of the coloured solver (96 bytes): J_l2 = -J_l1 for every row the
+// supported joints produce, the linear part of inv(M) J^T is the inverse mass
+// times that; the angular parts (inverse inertia times a1, a2) are kept.
 struct alignas(16) SRow {
   float l[3], a1[3], a2[3];
+  float t1[3], t2[3];
   float rhs, cfm, ad, lo, hi;
+  int findex;      // 0: friction bounded by the constraint's first row; -1: none
+  float im1, im2;  // inverse masses of the constraint's bodies
   float pad;
-  int findex;   // row (within its constraint) of the normal impulse, or -1
-};
-
-// per-body block of the coloured solver: fc (6), symmetric world inverse
-// inertia (xx xy xz yy yz zz), inverse mass, pad -- 64 bytes
-struct alignas(16) SBody {
-  float fc[6];
-  float iI[6];
-  float im;
-  float pad[3];
-};
-
-// per-body state of the accelerated coloured solver: fc before the sweep and
-// the search direction's fc (M^-1 J^T p)
-struct alignas(16) SAccBody {
-  float fp[6];
-  float fdir[6];
 };
 
 // per-constraint record of the coloured solver, constraints sorted by colour
@@ -198,7 +183,7 @@ enum { PH_AABB = 0, PH_BROAD, PH_NARROW, PH_BODIES, PH_ROWS, PH_ORDER, PH_SOR, P
 
 struct ScratchLayout {
   long long aabb, gbig, gidx, glevel, gdb, cells, ecount, pairs, pkeys, pcount, contacts, cons, rows, btmp,
-      order, adjs, adj, island, color, misc, sor, ref, total;
+      order, adjs, adj, island, color, misc, sor, total;
 };
 
 OD_HD inline long long od_align(long long x) { return (x + 255) & ~255LL; }
@@ -217,35 +202,40 @@ OD_HD inline long long warm_bytes(int kcap, int nj) { return od_align(24LL * kca
 OD_HD inline long long lcp_ws_floats(int m) { return 2LL * m * m + 7LL * m + 64; }
 
 // bytes of the coloured solver's working set held in LDS when its rows and
-// all of the conjugate-gradient state stay in global memory: bodies,
+// all of the conjugate-gradient state stay in global memory: the bodies' fc,
 // constraints in colour order, colour starts and row impulses
-OD_HD inline long long sor_lds_bytes_rows_cg_global(int nb, int nrows, int ncons) {
-  return (long long)sizeof(SBody) * nb + (long long)sizeof(SCons) * ncons +
-         ((4LL * (2LL * ncons + 8) + 15) & ~15LL) + ((4LL * nrows + 15) & ~15LL);
+OD_HD inline long long sor_lds_bytes_rows_cg_global(int nb, int nrows, int ncons, int ngroups) {
+  return ((24LL * nb + 15) & ~15LL) + (long long)sizeof(SCons) * ncons + ((4LL * (ngroups + 1LL) + 15) & ~15LL) +
+         ((4LL * nrows + 15) & ~15LL);
 }
 
 // ... with the rows' conjugate-gradient state in LDS too (the rows and the
 // bodies' conjugate-gradient state in global memory)
-OD_HD inline long long sor_lds_bytes_rows_acc_global(int nb, int nrows, int ncons, bool accel = false) {
-  return sor_lds_bytes_rows_cg_global(nb, nrows, ncons) + (accel ? (8LL * nrows + 15) & ~15LL : 0LL);
+OD_HD inline long long sor_lds_bytes_rows_acc_global(int nb, int nrows, int ncons, int ngroups, bool accel = false) {
+  return sor_lds_bytes_rows_cg_global(nb, nrows, ncons, ngroups) + (accel ? (8LL * nrows + 15) & ~15LL : 0LL);
 }
 
-// ... with the bodies' conjugate-gradient state in LDS too (the rows in
-// global memory)
-OD_HD inline long long sor_lds_bytes_rows_global(int nb, int nrows, int ncons, bool accel = false) {
-  return sor_lds_bytes_rows_acc_global(nb, nrows, ncons, accel) + (accel ? (long long)sizeof(SAccBody) * nb : 0LL);
+// ... with the bodies' conjugate-gradient state (fc before the sweep, and
+// the search direction's fc: M^-1 J^T p) in LDS too (the rows in global memory)
+OD_HD inline long long sor_lds_bytes_rows_global(int nb, int nrows, int ncons, int ngroups, bool accel = false) {
+  return sor_lds_bytes_rows_acc_global(nb, nrows, ncons, ngroups, accel) + (accel ? 48LL * nb : 0LL);
 }
 
 // the whole working set (rows first); copied to the LDS pool for the sweeps
 // when it fits
-OD_HD inline long long sor_lds_bytes(int nb, int nrows, int ncons, bool accel = false) {
-  return (long long)sizeof(SRow) * nrows + sor_lds_bytes_rows_global(nb, nrows, ncons, accel);
+OD_HD inline long long sor_lds_bytes(int nb, int nrows, int ncons, int ngroups, bool accel = false) {
+  return (long long)sizeof(SRow) * nrows + sor_lds_bytes_rows_global(nb, nrows, ncons, ngroups, accel);
 }
 
-// the same working set in the world's scratch
-OD_HD inline long long sor_bytes(int nb, int nrows, int ncons, bool accel = false) {
-  return sor_lds_bytes(nb, nrows, ncons, accel);
+// the same working set in the world's scratch (a constraint adds at most one
+// colour)
+OD_HD inline long long sor_bytes(int nb, int nrows, int ncons) {
+  return sor_lds_bytes(nb, nrows, ncons, 2 * ncons + 8, true);
 }
+
+// the reference order's solve in the world's scratch: the state (fc and
+// impulses), the schedule (9 ints a row) and two sides a row
+OD_HD inline long long ref_bytes(int nb, int nrows) { return 200LL * nrows + 28LL * nb + 128; }
 
 // Per-world scratch layout.  nb/ng/nj: world sizes; pcap (a power of two),
 // kcap, rcap: pair, contact and row capacities.  Every array the kernels
@@ -275,9 +265,9 @@ OD_HD inline ScratchLayout scratch_layout(int nb, int ng, int nj, int pcap, int 
   L.island = o;   o = od_align(o + 4LL * (6LL * nb + 2 * ncons + 3LL * ng + 16));
   L.color = o;    o = od_align(o + 4LL * (ncons + nb));
   L.misc = o;     o = od_align(o + 4LL * 64);
-  L.sor = o;      o = od_align(o + sor_bytes(nb, rcap, (int)ncons, true));
-  // the reference order's solve: 4 + 36 + 160 bytes per row, 28 per body
-  L.ref = o;      o = od_align(o + 200LL * rcap + 28LL * nb + 128);
+  // the solver's working set: one of the two orders'
+  const long long sb = sor_bytes(nb, rcap, (int)ncons), rb = ref_bytes(nb, rcap);
+  L.sor = o;      o = od_align(o + (sb > rb ? sb : rb));
   L.total = o;
   return L;
 }

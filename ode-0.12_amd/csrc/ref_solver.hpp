@@ -47,10 +47,6 @@ struct alignas(16) RefSide {
 // lf of a row without a friction index, and of a lane that writes nothing
 enum { REF_NO_FRICTION = -1, REF_IDLE = -2 };
 
-// a lane's LDS byte (what a function that is not inlined is told of the pool)
-typedef __attribute__((address_space(3))) char LdsChar;
-typedef __attribute__((address_space(3))) float LdsFloat;
-
 // Placement of the working set: everything in the LDS pool; the (read-only)
 // sides in global memory; sides and schedule in global memory (both are read
 // ahead of their level); everything in the world's scratch.
@@ -390,10 +386,15 @@ __device__ inline void ref_sweeps(const RefSched &W, const RefSide *sides, char 
 template <int PLACE>
 __device__ __attribute__((noinline)) void sor_reference(Row *rows, float *bt, const int *isl, char *gws, LdsChar *pool,
                                                         int nrows, int ngroups, int nb, int iters, Shared &sh) {
-  rows = as_global(rows);
-  bt = as_global(bt);
-  isl = as_global(isl);
-  gws = as_global(gws);
+  rows = uniform_global(rows);
+  bt = uniform_global(bt);
+  isl = uniform_global(isl);
+  gws = uniform_global(gws);
+  pool = uniform(pool);
+  nrows = uniform(nrows);
+  ngroups = uniform(ngroups);
+  nb = uniform(nb);
+  iters = uniform(iters);
   const int nt = blockDim.x, t = threadIdx.x, m = nrows;
   char *const lds = (char *)pool;
   const long long b0 = ref_state_bytes(m, nb), b1 = b0 + ref_sched_bytes(m, nb);
@@ -411,11 +412,11 @@ __device__ __attribute__((noinline)) void sor_reference(Row *rows, float *bt, co
     for (int it = 0; it < iters; it += 8) {
       ref_shuffle(W, isl, m, ngroups, it >> 3);
       bool solo;
-      const int D = ref_levels(W, rows, m, solo, sh);
+      const int D = uniform(ref_levels(W, rows, m, solo, sh));
       ref_sides<PLACE>(W, rows, sides, m, nb, at, at + 24 * (nb + 1));
       __syncthreads();
       const int total = D * min(8, iters - it);
-      if (solo) {
+      if (uniform(solo)) {
         if (t < 64) ref_sweeps<PLACE, true>(W, sides, gws, D, total);
       } else {
         ref_sweeps<PLACE, false>(W, sides, gws, D, total);

@@ -793,62 +793,40 @@ __device__ inline float row_residual(const Row *rows, int r, const float *fc) {
   return proj_residual(R.lambda, y / Aii, lo, hi);
 }
 
-// Coloured SOR-LCP.  The working set -- per-body fc, world inverse inertia
-// (symmetric) and inverse mass; the constraints sorted by colour with their
-// rows stored contiguously in that order -- is copied into the LDS pool when
-// it fits, else into the world's scratch.  One lane relaxes all rows of one
-// constraint with both bodies' fc in registers; the constraints of a colour
-// share no body, so a colour is one parallel pass.  Each row follows the
-// reference's update (quickstep.cpp:484-582) with inv(M) J^T rebuilt from
-// the body data (every supported row has J_lin2 = -J_lin1).
+// Coloured SOR-LCP.  The working set -- per-body fc; the constraints sorted
+// by colour with their rows stored contiguously in that order -- is copied
+// into the LDS pool as far as it fits, else stays in the world's scratch.
+// One lane relaxes all rows of one constraint with both bodies' fc in
+// registers; the constraints of a colour share no body, so a colour is one
+// parallel pass.  Each row follows the reference's update
+// (quickstep.cpp:484-582) on the inverse masses and the angular parts of
+// inv(M) J^T (every supported row has J_lin2 = -J_lin1).
 constexpr int SOR_MAX_ROWS = 6;   // rows of one constraint (contact 3, ball 3, hinge 6, hinge2 6)
 
 // J_1 . f1 (+ J_2 . f2) of one row (J_l2 = -J_l1), summed in the order written
-// Rows of the coloured solver's working set are stored with their four
-// 16-byte chunks rotated by ((r >> 1) & 3) for row r: neighbouring lanes read
-// rows 3 (contacts) or 1 apart, whose 64-byte starts fall on two LDS banks
-// only; the rotation spreads one chunk read of eight such lanes over all 32
-// banks.  The layout is the same in global scratch and in LDS.
-__device__ inline int srow_chunk(int r, int j) { return j ^ ((r >> 1) & 3); }
-
-__device__ inline void store_srow(SRow *base, int r, const SRow &v) {
-  char *dst = (char *)(base + r);
-  const char *src = (const char *)&v;
-  for (int j = 0; j < 4; j++) __builtin_memcpy(dst + 16 * srow_chunk(r, j), src + 16 * j, 16);
-}
-
-__device__ inline SRow load_srow(const SRow *base, int r) {
-  SRow v;
-  const char *src = (const char *)(base + r);
-  char *dst = (char *)&v;
-  for (int j = 0; j < 4; j++) __builtin_memcpy(dst + 16 * j, src + 16 * srow_chunk(r, j), 16);
-  return v;
-}
-
 __device__ inline float sor_dot(const SRow &r, const float *f1, bool two, const float *f2) {
-  float s = r.l[0] * f1[0] + r.l[1] * f1[1] + r.l[2] * f1[2] + r.a1[0] * f1[3] + r.a1[1] * f1[4] + r.a1[2] * f1[5];
-  if (two)
-    s += -r.l[0] * f2[0] - r.l[1] * f2[1] - r.l[2] * f2[2] + r.a2[0] * f2[3] + r.a2[1] * f2[4] + r.a2[2] * f2[5];
-  return s;
+  const float s = r.l[0] * f1[0] + r.l[1] * f1[1] + r.l[2] * f1[2] + r.a1[0] * f1[3] + r.a1[1] * f1[4] + r.a1[2] * f1[5];
+  const float s2 =
+      -r.l[0] * f2[0] - r.l[1] * f2[1] - r.l[2] * f2[2] + r.a2[0] * f2[3] + r.a2[1] * f2[4] + r.a2[2] * f2[5];
+  return two ? s + s2 : s;
 }
 
 // largest complementarity residual |lambda - clamp(lambda - (A lambda - b)_i / A_ii)|
 // over the rows of one constraint of the coloured solver (A_ii = w / ad)
-__device__ inline float sor_cons_residual(const SBody *sb, const SRow *sr, const float *slam, const SCons q,
+__device__ inline float sor_cons_residual(const float *fc, const SRow *sr, const float *slam, const SCons q,
                                           float sor_w) {
   float f1[6], f2[6];
-  for (int k = 0; k < 6; k++) f1[k] = sb[q.b1].fc[k];
   const bool two = q.b2 >= 0;
-  if (two)
-    for (int k = 0; k < 6; k++) f2[k] = sb[q.b2].fc[k];
-  float r = 0.f;
+  for (int k = 0; k < 6; k++) { f1[k] = fc[6 * q.b1 + k]; f2[k] = fc[6 * max(q.b2, 0) + k]; }
+  float r = 0.f, lam0 = 0.f;
   for (int k = 0; k < q.m; k++) {
-    const SRow w = load_srow(sr, q.row0 + k);
+    const SRow w = sr[q.row0 + k];
     const float lam = slam[q.row0 + k];
+    if (k == 0) lam0 = lam;
     const float y = sor_dot(w, f1, two, f2) + w.cfm * lam - w.rhs;
     float lo = w.lo, hi = w.hi;
     if (w.findex >= 0) {
-      hi = fabsf(w.hi * slam[q.row0 + w.findex]);
+      hi = fabsf(w.hi * lam0);
       lo = -hi;
     }
     r = fmaxf(r, proj_residual(lam, y * (w.ad / sor_w), lo, hi));
@@ -856,74 +834,33 @@ __device__ inline float sor_cons_residual(const SBody *sb, const SRow *sr, const
   return r;
 }
 
-// fc += delta * inv(M) J^T of one row for both bodies of its constraint
-__device__ inline void sor_push(const SRow &r, float delta, float im1, const float *iI1, float *f1, bool two,
-                                float im2, const float *iI2, float *f2) {
-  float d1 = delta * im1;
-  f1[0] += d1 * r.l[0]; f1[1] += d1 * r.l[1]; f1[2] += d1 * r.l[2];
-  f1[3] += delta * (iI1[0] * r.a1[0] + iI1[1] * r.a1[1] + iI1[2] * r.a1[2]);
-  f1[4] += delta * (iI1[1] * r.a1[0] + iI1[3] * r.a1[1] + iI1[4] * r.a1[2]);
-  f1[5] += delta * (iI1[2] * r.a1[0] + iI1[4] * r.a1[1] + iI1[5] * r.a1[2]);
-  if (two) {
-    float d2 = delta * im2;
-    f2[0] -= d2 * r.l[0]; f2[1] -= d2 * r.l[1]; f2[2] -= d2 * r.l[2];
-    f2[3] += delta * (iI2[0] * r.a2[0] + iI2[1] * r.a2[1] + iI2[2] * r.a2[2]);
-    f2[4] += delta * (iI2[1] * r.a2[0] + iI2[3] * r.a2[1] + iI2[4] * r.a2[2]);
-    f2[5] += delta * (iI2[2] * r.a2[0] + iI2[4] * r.a2[1] + iI2[5] * r.a2[2]);
+// fc += delta * inv(M) J^T of one row for both bodies of its constraint (f2
+// of a constraint with one body is not used)
+__device__ inline void sor_push(const SRow &r, float delta, float *f1, float *f2) {
+  const float d1 = delta * r.im1, d2 = delta * r.im2;
+  for (int k = 0; k < 3; k++) {
+    f1[k] += d1 * r.l[k];
+    f1[3 + k] += delta * r.t1[k];
+    f2[k] -= d2 * r.l[k];
+    f2[3 + k] += delta * r.t2[k];
   }
 }
 
-// Relaxes the rows of one constraint with one lane (quickstep.cpp:484-582):
-// both bodies' fc in registers, the rows read three at a time so that the
-// LDS latency is paid once per group of rows.  tol_mode: fc follows the
-// stored impulse.
-__device__ inline void sor_relax(SBody *__restrict__ sb, const SRow *__restrict__ sr, float *__restrict__ slam,
-                                 float2 *__restrict__ ld, const SCons q, bool accel, bool tol_mode) {
-  const bool two = q.b2 >= 0;
-  const SBody B1 = sb[q.b1];
-  SBody B2;
-  if (two) B2 = sb[q.b2];
-  float f1[6], iI1[6], f2[6], iI2[6], im2 = 0.f;
-  for (int k = 0; k < 6; k++) { f1[k] = B1.fc[k]; iI1[k] = B1.iI[k]; f2[k] = 0.f; iI2[k] = 0.f; }
-  const float im1 = B1.im;
-  if (two) {
-    for (int k = 0; k < 6; k++) { f2[k] = B2.fc[k]; iI2[k] = B2.iI[k]; }
-    im2 = B2.im;
-  }
-  float lam0 = 0.f;
-  for (int k0 = 0; k0 < q.m; k0 += 3) {
-    SRow R3[3];
-    float L3[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-      if (k0 + j < q.m) { R3[j] = load_srow(sr, q.row0 + k0 + j); L3[j] = slam[q.row0 + k0 + j]; }
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      const int k = k0 + j;
-      if (k >= q.m) break;
-      const SRow &r = R3[j];
-      const float s = sor_dot(r, f1, two, f2);
-      const float old = L3[j];
-      if (accel) ld[q.row0 + k].x = old;
-      float delta = r.ad * (r.rhs - old * r.cfm - s);
-      float lo = r.lo, hi = r.hi;
-      if (r.findex >= 0) {
-        float ln = (r.findex == 0) ? lam0 : slam[q.row0 + r.findex];
-        hi = fabsf(r.hi * ln);
-        lo = -hi;
-      }
-      float nl = old + delta;
-      if (nl < lo) { delta = lo - old; nl = lo; }
-      else if (nl > hi) { delta = hi - old; nl = hi; }
-      else if (tol_mode) delta = nl - old;
-      slam[q.row0 + k] = nl;
-      if (k == 0) lam0 = nl;
-      sor_push(r, delta, im1, iI1, f1, two, im2, iI2, f2);
-    }
-  }
-  for (int k = 0; k < 6; k++) sb[q.b1].fc[k] = f1[k];
-  if (two)
-    for (int k = 0; k < 6; k++) sb[q.b2].fc[k] = f2[k];
+// One row (quickstep.cpp:484-582): its new impulse; f1, f2 follow.  lam0: the
+// impulse of the constraint's first row; tol_mode: fc follows the stored
+// impulse.  Free of branches, so that the two bodies' chains overlap.
+__device__ inline float sor_relax_row(const SRow &r, float old, float lam0, bool two, float *f1, float *f2,
+                                      bool tol_mode) {
+  const float s = sor_dot(r, f1, two, f2);
+  float delta = r.ad * (r.rhs - old * r.cfm - s);
+  const bool fr = r.findex >= 0;
+  const float hf = fabsf(r.hi * lam0), hi = fr ? hf : r.hi, lo = fr ? -hf : r.lo;
+  float nl = old + delta;
+  const bool below = nl < lo, above = !below && nl > hi;
+  nl = below ? lo : (above ? hi : nl);
+  delta = tol_mode || below || above ? nl - old : delta;
+  sor_push(r, delta, f1, f2);
+  return nl;
 }
 
 // Starting impulses of one constraint's rows from the warm-start records of
@@ -950,42 +887,50 @@ __device__ inline void warm_lookup(const WorldParams &P, const Cons &q, const Co
 }
 
 // The coloured solver's working set: the rows (read-only during the sweeps),
-// bodies, constraints in colour order, colour starts, the row impulses and
-// (accelerated mode) the conjugate-gradient state: per row lambda before the
-// sweep and the direction, per body fc before the sweep and the direction's
-// fc (last, so that a pool can hold all but it).  Built in the world's
-// scratch; copied to the LDS pool for the sweeps when it fits there (same
-// layout).
+// the bodies' fc, constraints in colour order, colour starts, the row impulses
+// and (accelerated mode) the conjugate-gradient state: per row lambda before
+// the sweep and the direction, per body fc before the sweep and the
+// direction's fc (last, so that a pool can hold all but it).  Built in the
+// world's scratch; copied to the LDS pool for the sweeps when it fits there
+// (same layout).
 struct SorSet {
   SRow *sr;
-  SBody *sb;
+  float *fc;
   SCons *sc;
   int *sstart;
   float *slam;
-  SAccBody *sa;
   float2 *ld;
+  float *fp, *fdir;
 };
 
-__device__ inline SorSet sor_set(char *base, SRow *sr, int nb, int nrows, int nact) {
+__device__ inline SorSet sor_set(char *base, SRow *sr, int nb, int nrows, int nact, int ngroups) {
   SorSet S;
   S.sr = sr;
-  S.sb = (SBody *)base;
-  S.sc = (SCons *)(S.sb + nb);
+  S.fc = (float *)base;
+  S.sc = (SCons *)(base + ((24LL * nb + 15) & ~15LL));
   S.sstart = (int *)(S.sc + nact);
-  S.slam = (float *)((char *)S.sstart + ((4LL * (2LL * nact + 8) + 15) & ~15LL));
+  S.slam = (float *)((char *)S.sstart + ((4LL * (ngroups + 1LL) + 15) & ~15LL));
   S.ld = (float2 *)((char *)S.slam + ((4LL * nrows + 15) & ~15LL));
-  S.sa = (SAccBody *)((char *)S.ld + ((8LL * nrows + 15) & ~15LL));
+  S.fp = (float *)((char *)S.ld + ((8LL * nrows + 15) & ~15LL));
+  S.fdir = S.fp + 6 * nb;
   return S;
 }
 
-__device__ inline SorSet sor_global(const Ctx &c, int nrows, int nact) {
+__device__ inline SorSet sor_global(const Ctx &c, int nrows, int nact, int ngroups) {
   SRow *sr = c.at<SRow>(c.L.sor);
-  return sor_set((char *)(sr + nrows), sr, c.W.nb, nrows, nact);
+  return sor_set((char *)(sr + nrows), sr, c.W.nb, nrows, nact, ngroups);
 }
 
 // per-world values handed from the solver's set-up to the sweeps and on to
 // the integration (split launches), in the world's misc block
 enum { MISC_SOR_ROWS = 8, MISC_SOR_GROUPS = 9, MISC_SOR_RESIDUAL = 10, MISC_SOR_READY = 11 };
+
+// inverse inertia (world, symmetric: its upper triangle) times a
+__device__ inline void sor_turn(const float *t, const float *a, float *o) {
+  o[0] = t[0] * a[0] + t[1] * a[1] + t[2] * a[2];
+  o[1] = t[1] * a[0] + t[4] * a[1] + t[5] * a[2];
+  o[2] = t[2] * a[0] + t[5] * a[1] + t[8] * a[2];
+}
 
 // Set-up: the working set in the world's scratch, in colour order, with the
 // starting impulses (zero, or the warm start from the previous step).
@@ -1001,16 +946,8 @@ __device__ void sor_prepare(const DevBatch &B, const Ctx &c, const WorldParams &
   const float *wjnt = warm_on ? (const float *)(B.warm + c.W.warm + od_align(24LL * c.W.kcap)) : nullptr;
   const ContactRec *con = c.at<ContactRec>(c.L.contacts);
   const int nt = blockDim.x;
-  const SorSet S = sor_global(c, nrows, nact);
-  for (int b = threadIdx.x; b < nb; b += nt) {
-    const float *t = bt + 32 * b;
-    SBody q;
-    for (int k = 0; k < 6; k++) q.fc[k] = 0.f;
-    q.iI[0] = t[0]; q.iI[1] = t[1]; q.iI[2] = t[2]; q.iI[3] = t[4]; q.iI[4] = t[5]; q.iI[5] = t[8];
-    q.im = B.invMass[c.W.b0 + b];
-    q.pad[0] = q.pad[1] = q.pad[2] = 0.f;
-    S.sb[b] = q;
-  }
+  const SorSet S = sor_global(c, nrows, nact, ngroups);
+  for (int e = threadIdx.x; e < 6 * nb; e += nt) S.fc[e] = 0.f;
   for (int k = threadIdx.x; k <= ngroups; k += nt) S.sstart[k] = cstart[k];
   int rbase = 0;
   for (int x0 = 0; x0 < nact; x0 += nt) {
@@ -1025,16 +962,21 @@ __device__ void sor_prepare(const DevBatch &B, const Ctx &c, const WorldParams &
       S.sc[x] = o;
       float wl[SOR_MAX_ROWS] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (warm) warm_lookup(P, *q, con, wrec, nprev, wjnt, wl);
+      const int b2 = max(o.b2, 0);
+      const float *t1 = bt + 32 * o.b1, *t2 = bt + 32 * b2;
+      const float im1 = B.invMass[c.W.b0 + o.b1], im2 = B.invMass[c.W.b0 + b2];
       for (int k = 0; k < m; k++) {
         const Row &R = rows[q->row0 + k];
         SRow w;
-        w.l[0] = R.J[0]; w.l[1] = R.J[1]; w.l[2] = R.J[2];
-        w.a1[0] = R.J[3]; w.a1[1] = R.J[4]; w.a1[2] = R.J[5];
-        w.a2[0] = R.J[9]; w.a2[1] = R.J[10]; w.a2[2] = R.J[11];
+        for (int j = 0; j < 3; j++) {
+          w.l[j] = R.J[j]; w.a1[j] = R.J[3 + j]; w.a2[j] = R.J[9 + j];
+        }
+        sor_turn(t1, w.a1, w.t1);
+        sor_turn(t2, w.a2, w.t2);
         w.rhs = R.rhs; w.cfm = R.cfm; w.ad = R.ad; w.lo = R.lo; w.hi = R.hi;
-        w.pad = 0.f;
-        w.findex = R.findex >= 0 ? R.findex - q->row0 : -1;
-        store_srow(S.sr, o.row0 + k, w);
+        w.im1 = im1; w.im2 = im2; w.pad = 0.f;
+        w.findex = R.findex >= 0 ? 0 : -1;
+        S.sr[o.row0 + k] = w;
         S.slam[o.row0 + k] = k < SOR_MAX_ROWS ? wl[k] : 0.f;
       }
     }
@@ -1048,47 +990,76 @@ __device__ void sor_prepare(const DevBatch &B, const Ctx &c, const WorldParams &
 // in the pool, everything but the rows and the bodies' conjugate-gradient
 // state (read and written once per sweep, by one coalesced pass) in the
 // pool, or also the rows' conjugate-gradient state in global scratch (inside
-// the colour chain a relaxation only stores to it).
-enum { SOR_IN_GLOBAL = 0, SOR_IN_LDS = 1, SOR_ROWS_GLOBAL = 2, SOR_ROWS_ACC_GLOBAL = 3, SOR_ROWS_CG_GLOBAL = 4 };
+// the colour chain a relaxation only stores to it), or the fc alone in the
+// pool (large worlds: it is all that one relaxation hands to another).
+enum {
+  SOR_IN_GLOBAL = 0, SOR_IN_LDS = 1, SOR_ROWS_GLOBAL = 2, SOR_ROWS_ACC_GLOBAL = 3, SOR_ROWS_CG_GLOBAL = 4,
+  SOR_FC_LDS = 5
+};
 
 // The sweeps.  The working set (rows included, or all but the rows) is
 // copied to the LDS pool first and back at the end; the placement is a
 // template argument so that every access compiles to LDS (or global)
 // instructions rather than generic flat ones.  Writes the iteration count
 // and leaves the last residual in the world's misc block.
+//
+// One pass relaxes up to blockDim.x constraints of a colour, one per lane,
+// with the fc of both bodies in registers.  Its chain (read fc, three rows of
+// two dot products and a clamp each, write fc, barrier) and its number of
+// instructions bound a sweep, the 0.8 TB/s of rows do not.  So a relaxation
+// has no branches inside a row and reads inv(M) J^T instead of multiplying it
+// out (96 bytes a row for 64, and no inertia in LDS); a row's successor is
+// loaded as soon as the row is done, which hides its latency behind one pass
+// without a second set of registers; and the barrier between colours orders
+// LDS only (the loads stay in flight) unless the fc are in global memory.
+// Two sets of rows in turn, loaded a pass ahead, spilled: 40 % slower than
+// this.  2048 uneven worlds, 64 lanes each: 20.7 -> 16.1 us a sweep of 816
+// rows at 20 sweeps, 150 -> 95 ms a step at a tolerance of 1e-4.
 template <bool TOL, int PLACE>
-__device__ __attribute__((always_inline)) void sor_solve(const DevBatch &B, const Ctx &c, const WorldParams &P,
-                                                         int nrows, int ngroups, int nact, bool host_contacts,
-                                                         Shared &sh) {
-  constexpr bool LDS = PLACE != SOR_IN_GLOBAL;
+__device__ __attribute__((noinline)) void sor_solve(char *gsor, int *cnt, int *misc, const WorldParams *Pg,
+                                                    LdsChar *pool, int nb, int nrows, int ngroups, int nact, bool warm,
+                                                    Shared &sh) {
+  constexpr bool IN_POOL = PLACE != SOR_IN_GLOBAL && PLACE != SOR_FC_LDS;
   constexpr bool ROWS_LDS = PLACE == SOR_IN_LDS;
-  const int nb = c.W.nb;
-  const bool use_tol = TOL && P.tol > 0.f;
-  const bool accel = use_tol && P.accel != 0;
-  const bool warm = P.warm != 0.f && !host_contacts && B.warm_n != nullptr && B.warm_n[c.w] >= 0;
+  gsor = uniform_global(gsor);
+  cnt = uniform_global(cnt);
+  misc = uniform_global(misc);
+  pool = uniform(pool);
+  nb = uniform(nb);
+  nrows = uniform(nrows);
+  ngroups = uniform(ngroups);
+  nact = uniform(nact);
+  warm = uniform(warm);
+  const WorldParams &P = *uniform_global(Pg);
+  const float tol = uniform(P.tol), sor_w = uniform(P.sor_w);
+  const bool use_tol = TOL && tol > 0.f;
+  const bool accel = use_tol && uniform(P.accel) != 0;
   const int nt = blockDim.x;
-  const SorSet G = sor_global(c, nrows, nact);
-  const SorSet S = ROWS_LDS ? sor_set((char *)((SRow *)od_pool + nrows), (SRow *)od_pool, nb, nrows, nact)
-                 : LDS      ? sor_set((char *)od_pool, G.sr, nb, nrows, nact)
-                            : G;
-  SRow *__restrict__ sr = S.sr;
-  SBody *__restrict__ sb = S.sb;
+  SRow *const grow = (SRow *)gsor;
+  const SorSet G = sor_set((char *)(grow + nrows), grow, nb, nrows, nact, ngroups);
+  char *const lds = (char *)pool;
+  const SorSet S = ROWS_LDS  ? sor_set((char *)((SRow *)lds + nrows), (SRow *)lds, nb, nrows, nact, ngroups)
+                   : IN_POOL ? sor_set(lds, G.sr, nb, nrows, nact, ngroups)
+                             : G;
+  SRow *__restrict__ sr = ROWS_LDS ? S.sr : G.sr;
+  float *__restrict__ fc = PLACE == SOR_FC_LDS ? (float *)lds : S.fc;
   SCons *__restrict__ sc = S.sc;
   int *__restrict__ sstart = S.sstart;
   float *__restrict__ slam = S.slam;
-  SAccBody *__restrict__ sa = PLACE >= SOR_ROWS_ACC_GLOBAL ? G.sa : S.sa;
-  float2 *__restrict__ ld = PLACE == SOR_ROWS_CG_GLOBAL ? G.ld : S.ld;
-  if (LDS) {
+  float *__restrict__ fp = PLACE >= SOR_ROWS_ACC_GLOBAL ? G.fp : S.fp;
+  float *__restrict__ fdir = PLACE >= SOR_ROWS_ACC_GLOBAL ? G.fdir : S.fdir;
+  float2 *__restrict__ ld = PLACE >= SOR_ROWS_CG_GLOBAL ? G.ld : S.ld;
+  if (IN_POOL) {
     if (ROWS_LDS)
-      for (int r = threadIdx.x; r < nrows; r += nt) sr[r] = G.sr[r];
-    for (int b = threadIdx.x; b < nb; b += nt) sb[b] = G.sb[b];
+      for (int e = threadIdx.x; e < 6 * nrows; e += nt) ((float4 *)sr)[e] = ((const float4 *)G.sr)[e];
     for (int x = threadIdx.x; x < nact; x += nt) sc[x] = G.sc[x];
     for (int k = threadIdx.x; k <= ngroups; k += nt) sstart[k] = G.sstart[k];
     for (int r = threadIdx.x; r < nrows; r += nt) slam[r] = G.slam[r];
   }
+  if (PLACE != SOR_IN_GLOBAL)
+    for (int e = threadIdx.x; e < 6 * nb; e += nt) fc[e] = 0.f;
   if (accel) {
-    for (int b = threadIdx.x; b < nb; b += nt)
-      for (int k = 0; k < 6; k++) { sa[b].fdir[k] = 0.f; sa[b].fp[k] = 0.f; }
+    for (int e = threadIdx.x; e < 6 * nb; e += nt) fdir[e] = fp[e] = 0.f;
     for (int r = threadIdx.x; r < nrows; r += nt) ld[r] = make_float2(0.f, 0.f);
   }
   __syncthreads();
@@ -1100,25 +1071,117 @@ __device__ __attribute__((always_inline)) void sor_solve(const DevBatch &B, cons
       for (int x = sstart[g] + threadIdx.x; x < x1; x += nt) {
         const SCons q = sc[x];
         const bool two = q.b2 >= 0;
-        float f1[6], f2[6] = {0, 0, 0, 0, 0, 0}, iI2[6] = {0, 0, 0, 0, 0, 0}, im2 = 0.f;
-        for (int k = 0; k < 6; k++) f1[k] = sb[q.b1].fc[k];
-        if (two)
-          for (int k = 0; k < 6; k++) { f2[k] = sb[q.b2].fc[k]; iI2[k] = sb[q.b2].iI[k]; }
-        if (two) im2 = sb[q.b2].im;
-        float iI1[6];
-        for (int k = 0; k < 6; k++) iI1[k] = sb[q.b1].iI[k];
-        const float im1 = sb[q.b1].im;
+        float f1[6], f2[6], *F1 = fc + 6 * q.b1, *F2 = fc + 6 * max(q.b2, 0);
+        for (int k = 0; k < 6; k++) { f1[k] = F1[k]; f2[k] = F2[k]; }
         for (int k = 0; k < q.m && k < SOR_MAX_ROWS; k++) {
           const float lam = slam[q.row0 + k];
-          if (lam != 0.f) sor_push(load_srow(sr, q.row0 + k), lam, im1, iI1, f1, two, im2, iI2, f2);
+          if (lam != 0.f) sor_push(sr[q.row0 + k], lam, f1, f2);
         }
-        for (int k = 0; k < 6; k++) sb[q.b1].fc[k] = f1[k];
+        for (int k = 0; k < 6; k++) F1[k] = f1[k];
         if (two)
-          for (int k = 0; k < 6; k++) sb[q.b2].fc[k] = f2[k];
+          for (int k = 0; k < 6; k++) F2[k] = f2[k];
       }
       __syncthreads();
     }
   }
+  // The passes of a sweep, in order and over again: [x0, x1) of a colour,
+  // whether the pass ends its colour and the sweep.  The end of the next
+  // colour is read a pass before it is needed.
+  struct Pass {
+    int x0;
+    bool colour_end, sweep_end;
+  };
+  int px0 = 0, px1 = 0, pg = ngroups - 1;   // the pass given out last and its colour; start as before colour 0
+  int pend = ngroups > 0 ? sstart[1] : 0;   // end of the colour after pg
+  auto next_pass = [&](SCons &q) -> Pass {
+    if (px0 + nt < px1) {
+      px0 += nt;
+    } else {
+      pg = pg + 1 == ngroups ? 0 : pg + 1;
+      px0 = pg == 0 ? 0 : px1;
+      px1 = __builtin_amdgcn_readfirstlane(pend);
+      pend = sstart[(pg + 1 == ngroups ? 0 : pg + 1) + 1];
+    }
+    const int x = px0 + (int)threadIdx.x;
+    q = sc[min(x, nact - 1)];
+    if (x >= px1) q.m = 0;
+    Pass v;
+    v.x0 = px0;
+    v.colour_end = px0 + nt >= px1;
+    v.sweep_end = v.colour_end && pg == ngroups - 1;
+    return v;
+  };
+  // The lane's three rows in hand and their impulses.  As soon as a row is
+  // relaxed the one that takes its place is loaded: the third row after it in
+  // a joint of more than three, else the next pass's.  (A lane without a
+  // constraint, or with fewer rows, loads a row that exists: one path for all
+  // lanes.)
+  SRow r[3];
+  float lam[3];
+  auto first_row = [&](const SCons &c, int j) { return c.row0 + max(0, min(j, c.m - 1)); };
+  SCons q, qn;    // the lane's constraint in this pass and in the next
+  Pass pc, pn;
+  if (nact > 0) {
+    pc = next_pass(q);
+#pragma unroll
+    for (int j = 0; j < 3; j++) { r[j] = sr[first_row(q, j)]; lam[j] = slam[first_row(q, j)]; }
+    pn = next_pass(qn);
+  }
+  auto reload_lam = [&] {
+    if (nact > 0)
+#pragma unroll
+      for (int j = 0; j < 3; j++) lam[j] = slam[first_row(q, j)];
+  };
+  // relaxes the pass; true at the sweep's end
+  auto pass = [&]() -> bool {
+    const bool on = q.m > 0, two = on && q.b2 >= 0;
+    float f1[6], f2[6], *F1 = fc + 6 * q.b1, *F2 = fc + 6 * max(q.b2, 0);
+    for (int k = 0; k < 6; k++) { f1[k] = F1[k]; f2[k] = F2[k]; }
+    const Pass nx = pn;
+    SCons q2;
+    pn = next_pass(q2);
+    float lam0 = 0.f;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int i = q.row0 + j;
+      if (j < q.m) {
+        if (accel) ld[i].x = lam[j];
+        lam[j] = sor_relax_row(r[j], lam[j], lam0, two, f1, f2, use_tol);
+        slam[i] = lam[j];
+        if (j == 0) lam0 = lam[j];
+      }
+      const int n = 3 + j < q.m ? i + 3 : first_row(qn, j);
+      r[j] = sr[n];
+      lam[j] = slam[n];
+    }
+    for (int k0 = 3; k0 < q.m; k0 += 3) {
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        const int i = q.row0 + k0 + j;
+        if (k0 + j < q.m) {
+          if (accel) ld[i].x = lam[j];
+          slam[i] = sor_relax_row(r[j], lam[j], lam0, two, f1, f2, use_tol);
+          const int n = k0 + 3 + j < q.m ? i + 3 : first_row(qn, j);
+          r[j] = sr[n];
+          lam[j] = slam[n];
+        }
+      }
+    }
+    if (on)
+      for (int k = 0; k < 6; k++) F1[k] = f1[k];
+    if (two)
+      for (int k = 0; k < 6; k++) F2[k] = f2[k];
+    const Pass done = pc;
+    pc = nx;
+    q = qn;
+    qn = q2;
+    if (done.colour_end) {
+      // the end of a sweep hands on impulses and directions too
+      if (PLACE == SOR_IN_GLOBAL || done.sweep_end) __syncthreads();
+      else lds_barrier();
+    }
+    return done.sweep_end;
+  };
   // fixed iteration count, or (tol > 0) iterate until the LCP residual of
   // the world is at most tol, checked every check_every iterations, up to
   // max_iterations; accelerated: between sweeps a nonsmooth nonlinear
@@ -1127,8 +1190,8 @@ __device__ __attribute__((always_inline)) void sor_solve(const DevBatch &B, cons
   // lambda += beta p_prev (applied before the next sweep, so the solver
   // always ends on a projected sweep), p = d + beta p_prev; fc follows
   // through M^-1 J^T p
-  const int maxit = use_tol ? P.max_iterations : P.iterations;
-  const int every = use_tol ? (P.check_every > 0 ? P.check_every : 1) : (maxit > 0 ? maxit : 1);
+  const int maxit = uniform(use_tol ? P.max_iterations : P.iterations);
+  const int every = uniform(use_tol ? (P.check_every > 0 ? P.check_every : 1) : (maxit > 0 ? maxit : 1));
   float rr_prev = 0.f, res_prev = INFINITY;
   bool acc = accel;        // CG steps still on for this solve
   float res_last = 0.f;    // residual at the last check
@@ -1143,27 +1206,22 @@ __device__ __attribute__((always_inline)) void sor_solve(const DevBatch &B, cons
         // into the previous sweep's CG update below
         for (int r = threadIdx.x; r < nrows; r += nt)
           if (ld[r].x != 0.f) slam[r] += ld[r].x;
-        for (int e = threadIdx.x; e < 6 * nb; e += nt) {   // one fc component per lane
-          const int b = e / 6, k = e - 6 * b;
-          sb[b].fc[k] += sa[b].fp[k];
-          sa[b].fp[k] = sb[b].fc[k];
-        }
+        for (int e = threadIdx.x; e < 6 * nb; e += nt) fp[e] = fc[e] += fp[e];   // one fc component per lane
         __syncthreads();
+        reload_lam();
       }
-      for (int g = 0; g < ngroups; g++) {
-        const int x1 = sstart[g + 1];
-        for (int x = sstart[g] + threadIdx.x; x < x1; x += nt) sor_relax(sb, sr, slam, ld, sc[x], accel, use_tol);
-        __syncthreads();
-      }
+      if (nact > 0)
+        while (!pass()) {}
       if (acc) {
         // d = this sweep's change; beta = |d|^2 / |d_prev|^2 (restart when
         // > 1); the momentum beta p_prev is applied before the next sweep
         float loc = 0.f;
+#pragma unroll 4
         for (int r = threadIdx.x; r < nrows; r += nt) {
           float d = slam[r] - ld[r].x;
           loc += d * d;
         }
-        const float rr = block_fsum(loc, sh);
+        const float rr = uniform(block_fsum(loc, sh));
         float beta = (rr_prev > 0.f) ? rr / rr_prev : 0.f;
         if (!(beta <= 1.f)) beta = 0.f;
         // the next sweep of this block takes the momentum now (the same
@@ -1171,123 +1229,96 @@ __device__ __attribute__((always_inline)) void sor_solve(const DevBatch &B, cons
         // before a check leaves it pending, so the check sees the sweep's
         // own result
         const bool now = rep + 1 < n;
+#pragma unroll 4
         for (int r = threadIdx.x; r < nrows; r += nt) {
-          float d = slam[r] - ld[r].x;
-          float pend = beta * ld[r].y;   // momentum along the previous direction
-          ld[r].y = d + pend;            // new direction
-          if (!now) ld[r].x = pend;
-          else if (pend != 0.f) slam[r] += pend;
+          const float2 o = ld[r];
+          const float lam = slam[r], d = lam - o.x;
+          const float pend = beta * o.y;                             // momentum along the previous direction
+          ld[r] = make_float2(now ? o.x : pend, d + pend);           // and the new direction
+          if (now) slam[r] = pend != 0.f ? lam + pend : lam;
         }
         for (int e = threadIdx.x; e < 6 * nb; e += nt) {   // one fc component per lane
-          const int b = e / 6, k = e - 6 * b;
-          float pend = beta * sa[b].fdir[k];
-          sa[b].fdir[k] = (sb[b].fc[k] - sa[b].fp[k]) + pend;
-          if (!now) {
-            sa[b].fp[k] = pend;
-          } else {
-            sb[b].fc[k] += pend;
-            sa[b].fp[k] = sb[b].fc[k];
-          }
+          const float f = fc[e], pend = beta * fdir[e];
+          fdir[e] = (f - fp[e]) + pend;
+          fp[e] = now ? f + pend : pend;
+          if (now) fc[e] = f + pend;
         }
         rr_prev = rr;
         __syncthreads();
+        reload_lam();
       }
     }
     it += n;
     if (use_tol) {
       float r = 0.f;
-      for (int x = threadIdx.x; x < nact; x += nt) r = fmaxf(r, sor_cons_residual(sb, sr, slam, sc[x], P.sor_w));
-      r = block_max(r, sh);
+      for (int x = threadIdx.x; x < nact; x += nt) r = fmaxf(r, sor_cons_residual(fc, sr, slam, sc[x], sor_w));
+      r = uniform(block_max(r, sh));
       res_last = r;
-      if (r <= P.tol) break;
+      if (r <= tol) break;
       if (acc && !(r <= res_prev)) {
         // the residual rose since the last check: restart the CG steps, and
         // stop them for the rest of the solve when the residual is still far
         // (> 1000 tol) from the tolerance
         for (int q = threadIdx.x; q < nrows; q += nt) ld[q] = make_float2(0.f, 0.f);
-        for (int b = threadIdx.x; b < nb; b += nt)
-          for (int k = 0; k < 6; k++) { sa[b].fdir[k] = 0.f; sa[b].fp[k] = 0.f; }
+        for (int e = threadIdx.x; e < 6 * nb; e += nt) fdir[e] = fp[e] = 0.f;
         rr_prev = 0.f;
-        if (r > 1000.f * P.tol) acc = false;
+        if (r > 1000.f * tol) acc = false;
         __syncthreads();
       }
       res_prev = r;
     }
   }
   if (threadIdx.x == 0) {
-    B.counters[c.w * CNT_N + CNT_ITERS] = it;
-    c.at<int>(c.L.misc)[MISC_SOR_RESIDUAL] = __float_as_int(use_tol ? res_last : 0.f);
+    cnt[CNT_ITERS] = it;
+    misc[MISC_SOR_RESIDUAL] = __float_as_int(use_tol ? res_last : 0.f);
     if (use_tol) {
-      int *cw = B.counters + c.w * CNT_N;
-      if (!(res_last <= P.tol)) cw[CNT_UNCONV] += 1;
+      if (!(res_last <= tol)) cnt[CNT_UNCONV] += 1;
       // non-negative floats order like their bit patterns
       const int rb = __float_as_int(res_last == res_last ? res_last : INFINITY);
-      if (rb > cw[CNT_RESMAX]) cw[CNT_RESMAX] = rb;
+      if (rb > cnt[CNT_RESMAX]) cnt[CNT_RESMAX] = rb;
     }
   }
-  if (LDS) {
-    for (int b = threadIdx.x; b < nb; b += nt)
-      for (int k = 0; k < 6; k++) G.sb[b].fc[k] = sb[b].fc[k];
-    for (int r = threadIdx.x; r < nrows; r += nt) G.slam[r] = slam[r];
+  if (PLACE != SOR_IN_GLOBAL) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < 6 * nb; e += nt) G.fc[e] = fc[e];
   }
+  if (IN_POOL)
+    for (int r = threadIdx.x; r < nrows; r += nt) G.slam[r] = slam[r];
   __syncthreads();
 }
 
-// the sweeps on the working set in global scratch (worlds larger than the LDS
-// pool); kept out of line so that the LDS variant is not merged with it
-template <bool TOL>
-__device__ __attribute__((noinline)) void sor_solve_global(const DevBatch &B, const Ctx &c, const WorldParams &P,
-                                                           int nrows, int ngroups, int nact, bool host_contacts,
-                                                           Shared &sh) {
-  sor_solve<TOL, SOR_IN_GLOBAL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-}
-
-// the sweeps with the rows read from global scratch and the rest of the
-// working set in the pool (worlds whose rows do not fit); out of line too
-template <bool TOL>
-__device__ __attribute__((noinline)) void sor_solve_rows_global(const DevBatch &B, const Ctx &c,
-                                                                const WorldParams &P, int nrows, int ngroups,
-                                                                int nact, bool host_contacts, Shared &sh) {
-  sor_solve<TOL, SOR_ROWS_GLOBAL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-}
-
-template <bool TOL>
-__device__ __attribute__((noinline)) void sor_solve_rows_acc_global(const DevBatch &B, const Ctx &c,
-                                                                    const WorldParams &P, int nrows, int ngroups,
-                                                                    int nact, bool host_contacts, Shared &sh) {
-  sor_solve<TOL, SOR_ROWS_ACC_GLOBAL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-}
-
-template <bool TOL>
-__device__ __attribute__((noinline)) void sor_solve_rows_cg_global(const DevBatch &B, const Ctx &c,
-                                                                   const WorldParams &P, int nrows, int ngroups,
-                                                                   int nact, bool host_contacts, Shared &sh) {
-  sor_solve<TOL, SOR_ROWS_CG_GLOBAL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-}
-
+// the placement with as much as fits in `lds` bytes of the pool
 template <bool TOL>
 __device__ inline void sor_solve_any(const DevBatch &B, const Ctx &c, const WorldParams &P, int nrows, int ngroups,
-                                     int nact, bool host_contacts, Shared &sh) {
+                                     int nact, bool host_contacts, int lds, Shared &sh) {
+  const int nb = c.W.nb;
   const bool accel = TOL && P.tol > 0.f && P.accel != 0;
-  if (sor_lds_bytes(c.W.nb, nrows, nact, accel) <= B.lds_bytes)
-    sor_solve<TOL, SOR_IN_LDS>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-  else if (sor_lds_bytes_rows_global(c.W.nb, nrows, nact, accel) <= B.lds_bytes)
-    sor_solve_rows_global<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-  else if (accel && sor_lds_bytes_rows_acc_global(c.W.nb, nrows, nact, accel) <= B.lds_bytes)
-    sor_solve_rows_acc_global<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-  else if (accel && sor_lds_bytes_rows_cg_global(c.W.nb, nrows, nact) <= B.lds_bytes)
-    sor_solve_rows_cg_global<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
+  const bool warm = P.warm != 0.f && !host_contacts && B.warm_n != nullptr && B.warm_n[c.w] >= 0;
+  char *gsor = c.at<char>(c.L.sor);
+  int *cnt = B.counters + c.w * CNT_N, *misc = c.at<int>(c.L.misc);
+  LdsChar *pool = (LdsChar *)od_pool;
+  if (sor_lds_bytes(nb, nrows, nact, ngroups, accel) <= lds)
+    sor_solve<TOL, SOR_IN_LDS>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
+  else if (sor_lds_bytes_rows_global(nb, nrows, nact, ngroups, accel) <= lds)
+    sor_solve<TOL, SOR_ROWS_GLOBAL>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
+  else if (accel && sor_lds_bytes_rows_acc_global(nb, nrows, nact, ngroups, accel) <= lds)
+    sor_solve<TOL, SOR_ROWS_ACC_GLOBAL>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
+  else if (accel && sor_lds_bytes_rows_cg_global(nb, nrows, nact, ngroups) <= lds)
+    sor_solve<TOL, SOR_ROWS_CG_GLOBAL>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
+  else if (24LL * nb <= lds)
+    sor_solve<TOL, SOR_FC_LDS>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
   else
-    sor_solve_global<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
+    sor_solve<TOL, SOR_IN_GLOBAL>(gsor, cnt, misc, &P, pool, nb, nrows, ngroups, nact, warm, sh);
 }
 
 // After the sweeps: impulses back to the rows (constraint order), fc to the
 // per-body scratch, and the warm-start records of the next step.
 __device__ void sor_finish(const DevBatch &B, const Ctx &c, const WorldParams &P, const Cons *cons, Row *rows,
-                           float *bt, const int *corder, int nrows, int nact, int nk, int ncons, bool host_contacts) {
+                           float *bt, const int *corder, int nrows, int nact, int ngroups, int nk, int ncons,
+                           bool host_contacts) {
   const int nb = c.W.nb;
   const int nt = blockDim.x;
-  const SorSet G = sor_global(c, nrows, nact);
+  const SorSet G = sor_global(c, nrows, nact, ngroups);
   const bool warm_on = P.warm != 0.f && !host_contacts && B.warm_n != nullptr;
   WarmRec *wrec = warm_on ? (WarmRec *)(B.warm + c.W.warm) : nullptr;
   float *wjnt = warm_on ? (float *)(B.warm + c.W.warm + od_align(24LL * c.W.kcap)) : nullptr;
@@ -1299,7 +1330,7 @@ __device__ void sor_finish(const DevBatch &B, const Ctx &c, const WorldParams &P
     for (int k = 0; k < o.m; k++) rows[q.row0 + k].lambda = G.slam[o.row0 + k];
   }
   for (int b = threadIdx.x; b < nb; b += nt)
-    for (int k = 0; k < 6; k++) bt[32 * b + 9 + k] = G.sb[b].fc[k];
+    for (int k = 0; k < 6; k++) bt[32 * b + 9 + k] = G.fc[6 * b + k];
   __syncthreads();
   const bool use_tol = P.tol > 0.f;
   if (warm_on && use_tol && !(res_last <= 100.f * P.tol)) {
@@ -1338,8 +1369,8 @@ __device__ void sor_colored(const DevBatch &B, const Ctx &c, const WorldParams &
                             int ncons, bool host_contacts, Shared &sh) {
   const int nact = cstart[ngroups];
   sor_prepare(B, c, P, cons, rows, bt, corder, cstart, nrows, ngroups, host_contacts, sh);
-  sor_solve_any<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, sh);
-  sor_finish(B, c, P, cons, rows, bt, corder, nrows, nact, nk, ncons, host_contacts);
+  sor_solve_any<TOL>(B, c, P, nrows, ngroups, nact, host_contacts, B.lds_bytes, sh);
+  sor_finish(B, c, P, cons, rows, bt, corder, nrows, nact, ngroups, nk, ncons, host_contacts);
 }
 
 // LDS bytes of the reference-order constraint ordering: 12 ints per
@@ -1519,12 +1550,12 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
     ngroups = misc[MISC_SOR_GROUPS];
     const int nact = isl[ngroups];
     const bool accel = TOL && P.tol > 0.f && P.accel != 0;
-    if (sor_lds_bytes(nb, nrows, nact, accel) > B.sor_lds_bytes) {
+    if (sor_lds_bytes(nb, nrows, nact, ngroups, accel) > B.sor_lds_bytes) {
       // not solved by the sweep kernel (its LDS pool is too small)
-      sor_solve_global<TOL>(B, c, P, nrows, ngroups, nact, in.from_host, sh);
+      sor_solve_any<TOL>(B, c, P, nrows, ngroups, nact, in.from_host, 0, sh);
       c.clk.lap(PH_SOR);
     }
-    sor_finish(B, c, P, cons, rows, bt, corder, nrows, nact, nk, ncons, in.from_host);
+    sor_finish(B, c, P, cons, rows, bt, corder, nrows, nact, ngroups, nk, ncons, in.from_host);
   } else {
   // --- bodies: world inverse inertia, gyroscopic torque, gravity
   //     (quickstep.cpp:609-665)
@@ -1984,7 +2015,7 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
   const int iters = P.iterations;
   if (ref) {
     // the placement with as much as fits in the LDS pool
-    char *gws = c.at<char>(c.L.ref);
+    char *gws = c.at<char>(c.L.sor);
     const long long st = ref_state_bytes(nrows, nb), sched = ref_sched_bytes(nrows, nb);
     if (P.exact && B.lcp_ws)
       lcp_exact_world(B, c.w, rows, bt, isl, ngroups, nb, sh);
@@ -2282,14 +2313,14 @@ __device__ void sor_world(const DevBatch &B, int w, Shared &sh) {
   const bool accel = TOL && P.tol > 0.f && P.accel != 0;
   // a world whose working set does not fit the pool is solved by the
   // integration kernel, in global scratch
-  if (sor_lds_bytes(c.W.nb, nrows, nact, accel) > B.lds_bytes) return;
+  if (sor_lds_bytes(c.W.nb, nrows, nact, ngroups, accel) > B.lds_bytes) return;
   c.clk.start(B, w);
-  sor_solve<TOL, SOR_IN_LDS>(B, c, P, nrows, ngroups, nact, false, sh);
+  sor_solve_any<TOL>(B, c, P, nrows, ngroups, nact, false, B.lds_bytes, sh);
   c.clk.lap(PH_SOR);
 }
 
 template <bool TOL>
-__global__ __launch_bounds__(WG) void sor_kernel(DevBatch B, int first_world, int persistent) {
+__global__ __launch_bounds__(WG, 2) void sor_kernel(DevBatch B, int first_world, int persistent) {
   __shared__ Shared sh;
   if (!persistent) {
     int w = first_world + blockIdx.x;
