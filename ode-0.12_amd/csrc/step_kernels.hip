@@ -84,20 +84,6 @@ __device__ inline int block_excl_scan(int v, int &total, Shared &sh) {
   return off + x - v;
 }
 
-// colouring: the lowest colour below 64 that neither body's mask (body temp
-// words 24-25) holds and that is not full; 64 if none
-__device__ inline int first_free_colour(const float *bt, int b1, int b2, unsigned long long full) {
-  const unsigned long long used = *(const unsigned long long *)(bt + 32 * b1 + 24) |
-                                  (b2 >= 0 ? *(const unsigned long long *)(bt + 32 * b2 + 24) : 0ull) | full;
-  return used == ~0ull ? 64 : __ffsll((long long)~used) - 1;
-}
-
-__device__ inline void take_colour(float *bt, int b1, int b2, int *col, int c) {
-  *col = c;
-  *(unsigned long long *)(bt + 32 * b1 + 24) |= 1ull << c;
-  if (b2 >= 0) *(unsigned long long *)(bt + 32 * b2 + 24) |= 1ull << c;
-}
-
 __device__ inline float block_max(float v, Shared &sh) {
   int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
@@ -764,6 +750,7 @@ __device__ inline Surf host_surface(const ContactIn &ci) {
   return s;
 }
 
+#include "colouring.hpp"
 #include "ref_solver.hpp"
 
 // |lambda - clamp(lambda - d, lo, hi)| evaluated without the cancellation of
@@ -1542,7 +1529,7 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
   const int ncons = nk + nj;
   int *corder = c.at<int>(c.L.order);          // constraint order (island order when ref)
   int *isl = c.at<int>(c.L.island);            // ref: [cons0, ncons, row0, nrows, seed] per island
-  int *color = c.at<int>(c.L.color);
+  int *color = c.at<int>(c.L.color);           // ref: body tags, then constraint tags and Info2 erp
   int nrows = 0, ngroups = 0;
   if (STAGE == 2) {
     if (misc[MISC_SOR_READY] == 0) return;     // the step left the world unchanged
@@ -1749,150 +1736,16 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
       r0 += tot;
     }
     nrows = r0;
-    // colouring: each round takes the constraints whose priority is the
-    // largest among the still uncoloured constraints at both their bodies;
-    // the round's winners share no body.  Working set in the LDS pool when
-    // it fits.
-    const bool in_lds = 4LL * (nb + 3LL * ncons) <= B.lds_bytes;
-    int *bmax = in_lds ? (int *)od_pool : c.at<int>(c.L.adjs);
-    int *col = in_lds ? bmax + nb : color;
-    int *cb1 = in_lds ? col + ncons : c.at<int>(c.L.adj);
-    int *cb2 = cb1 + ncons;
-    for (int i = threadIdx.x; i < ncons; i += blockDim.x) {
-      col[i] = (cons[i].m > 0) ? -1 : -2;
-      cb1[i] = cons[i].b1;
-      cb2[i] = cons[i].b2;
-    }
-    // per body: the colours taken by its coloured constraints (64-bit mask
-    // in the body's unused temp words 24-25)
-    for (int b = threadIdx.x; b < nb; b += blockDim.x) *(unsigned long long *)(bt + 32 * b + 24) = 0ull;
-    // members of each of the first 64 colours, and the mask of full ones
-    for (int k = threadIdx.x; k < 64; k += blockDim.x) sh.ccount[k] = 0;
-    if (threadIdx.x == 0) sh.ival[9] = sh.ival[10] = 0;
-    __syncthreads();
-    int round = 0;
-    while (true) {
-      for (int b = threadIdx.x; b < nb; b += blockDim.x) bmax[b] = -1;
-      __syncthreads();
-      int left = 0;
-      for (int i = threadIdx.x; i < ncons; i += blockDim.x) {
-        if (col[i] != -1) continue;
-        left++;
-        int pr = (int)(((unsigned)i * 2654435761u) & 0x7fffffffu);   // unique hashed priority
-        atomicMax(&bmax[cb1[i]], pr);
-        if (cb2[i] >= 0) atomicMax(&bmax[cb2[i]], pr);
-      }
-      int nleft = block_sum(left, sh);
-      if (nleft == 0) break;
-      for (int i = threadIdx.x; i < ncons; i += blockDim.x) {
-        if (col[i] != -1) continue;
-        int pr = (int)(((unsigned)i * 2654435761u) & 0x7fffffffu);
-        if (bmax[cb1[i]] == pr && (cb2[i] < 0 || bmax[cb2[i]] == pr)) col[i] = -3;   // a winner, colour pending
-      }
-      __syncthreads();
-      // first fit, capped: the winners, in constraint order, each take the
-      // lowest colour that neither body has taken and that has fewer than
-      // blockDim.x members (a colour is then one pass of the block); past 64
-      // colours, one colour of their own per round.  Colours are settled in
-      // increasing order: below the lowest colour the winners would overfill
-      // every proposal stands; that colour goes to its first proposers in
-      // constraint order and is full, and the rest propose again.  A
-      // winner's proposal only rises, and a round's winners share no body
-      // (each mask has one writer per round), so this equals the sequential
-      // assignment.
-      while (true) {
-        const unsigned long long full = ((unsigned long long)(unsigned)sh.ival[10] << 32) | (unsigned)sh.ival[9];
-        for (int k = threadIdx.x; k < 64; k += blockDim.x) sh.ccur[k] = 0;
-        __syncthreads();
-        for (int i = threadIdx.x; i < ncons; i += blockDim.x)
-          if (col[i] == -3) {
-            const int p = first_free_colour(bt, cb1[i], cb2[i], full);
-            if (p < 64) atomicAdd(&sh.ccur[p], 1);
-          }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-          int cs = 64;
-          for (int k = 0; k < 64; k++)
-            if (sh.ccount[k] + sh.ccur[k] > (int)blockDim.x) { cs = k; break; }
-          sh.ival[8] = cs;
-        }
-        __syncthreads();
-        const int cs = sh.ival[8];
-        for (int i = threadIdx.x; i < ncons; i += blockDim.x)
-          if (col[i] == -3) {
-            const int p = first_free_colour(bt, cb1[i], cb2[i], full);
-            if (p < cs) take_colour(bt, cb1[i], cb2[i], col + i, p);
-            else if (p >= 64) col[i] = 64 + round;
-          }
-        for (int k = threadIdx.x; k < cs; k += blockDim.x) sh.ccount[k] += sh.ccur[k];
-        if (cs == 64) break;
-        const int room = (int)blockDim.x - sh.ccount[cs];
-        int base = 0;
-        for (int start = 0; start < ncons && base < room; start += blockDim.x) {
-          const int i = start + threadIdx.x;
-          const bool want = i < ncons && col[i] == -3 && first_free_colour(bt, cb1[i], cb2[i], full) == cs;
-          int tot;
-          const int r = base + block_excl_scan(want ? 1 : 0, tot, sh);
-          if (want && r < room) take_colour(bt, cb1[i], cb2[i], col + i, cs);
-          base += tot;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-          sh.ccount[cs] = (int)blockDim.x;
-          if (cs < 32) sh.ival[9] |= (int)(1u << cs);
-          else sh.ival[10] |= (int)(1u << (cs - 32));
-        }
-        __syncthreads();
-      }
-      __syncthreads();
-      round++;
-    }
-    {
-      int mc = -1;
-      for (int i = threadIdx.x; i < ncons; i += blockDim.x) mc = max(mc, col[i]);
-      ngroups = (int)block_max((float)mc, sh) + 1;
-    }
-    // bucket constraints by colour, stably (index order inside a colour):
-    // the sweep result does not depend on the order inside a colour, but
-    // the block sums of the stopping test and the CG step do, so the
-    // layout is kept reproducible from run to run
-    int *cstart = c.at<int>(c.L.island);   // ngroups+1 starts
-    if (ngroups <= MAX_COLORS_LDS) {
-      for (int k = threadIdx.x; k <= ngroups; k += blockDim.x) sh.ccount[k] = 0;
-      __syncthreads();
-      for (int i = threadIdx.x; i < ncons; i += blockDim.x)
-        if (col[i] >= 0) atomicAdd(&sh.ccount[col[i] + 1], 1);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        for (int k = 0; k < ngroups; k++) sh.ccount[k + 1] += sh.ccount[k];
-        for (int k = 0; k <= ngroups; k++) cstart[k] = sh.ccount[k];
-      }
-      __syncthreads();
-      for (int k = threadIdx.x; k < ngroups; k += blockDim.x) sh.ccur[k] = sh.ccount[k];
-      __syncthreads();
-      for (int start = 0; start < ncons; start += blockDim.x) {
-        const int i = start + threadIdx.x;
-        const int ci = (i < ncons) ? col[i] : -1;
-        if (ci >= 0) {
-          int rank = 0;
-          for (int j = start; j < i; j++) rank += (col[j] == ci);
-          corder[sh.ccur[ci] + rank] = i;
-        }
-        __syncthreads();
-        if (ci >= 0) atomicAdd(&sh.ccur[ci], 1);
-        __syncthreads();
-      }
-    } else if (threadIdx.x == 0) {
-      for (int k = 0; k <= ngroups; k++) cstart[k] = 0;
-      for (int i = 0; i < ncons; i++)
-        if (col[i] >= 0) cstart[col[i] + 1]++;
-      for (int k = 0; k < ngroups; k++) cstart[k + 1] += cstart[k];
-      int *cur = cstart + ngroups + 1;
-      for (int k = 0; k < ngroups; k++) cur[k] = cstart[k];
-      for (int i = 0; i < ncons; i++)
-        if (col[i] >= 0) corder[cur[col[i]]++] = i;
-    }
-    __syncthreads();
+    int *bmax = c.at<int>(c.L.adjs), *lists = c.at<int>(c.L.sor);
+    LdsChar *pool = (LdsChar *)od_pool;
+    const long long cb = col_bodies_bytes(nb);
+    if (cb + col_lists_bytes(ncons) <= B.lds_bytes)
+      ngroups = colour_constraints<COL_IN_LDS>(cons, bt, bmax, lists, pool, nb, ncons, corder, isl, sh);
+    else if (cb <= B.lds_bytes)
+      ngroups = colour_constraints<COL_BODIES_LDS>(cons, bt, bmax, lists, pool, nb, ncons, corder, isl, sh);
+    else
+      ngroups = colour_constraints<COL_IN_GLOBAL>(cons, bt, bmax, lists, pool, nb, ncons, corder, isl, sh);
+    ngroups = uniform(ngroups);
   }
   c.clk.lap(PH_ORDER);
   if (nrows > c.W.rcap) {
