@@ -62,8 +62,7 @@ void refresh_dev(BatchImpl *b) {
   D.sor_lds_bytes = b->sor_lds;
 }
 
-// LDS limits of the current device and the default pool: half a CU's LDS
-// less the kernel's static block, so that two workgroups share a CU.
+// LDS limits of the current device.
 static void init_lds(BatchImpl *b, int dev) {
   int per_cu = 0, per_block = 0, khz = 0;
   if (hipDeviceGetAttribute(&per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
@@ -81,9 +80,44 @@ static void init_lds(BatchImpl *b, int dev) {
     (void)hipGetLastError();
     b->lds_max = ((per_block < 65536 ? per_block : 65536) - st) & ~255;
   }
-  int half = (per_cu / 2 - st - 256) & ~255;
-  b->lds = half < b->lds_max ? half : b->lds_max;
-  if (b->lds < 0) b->lds = 0;
+}
+
+// the pool of k workgroups on a CU
+static int lds_share(const BatchImpl *b, int k) {
+  const int lds = (b->lds_cu / k - world_kernel_static_lds() - 256) & ~255;
+  return lds < 0 ? 0 : (lds < b->lds_max ? lds : b->lds_max);
+}
+
+// The launch shape until one is set or tuned, by the number of worlds N, the
+// CUs and the worlds' size.  The kernel leaves a SIMD two wavefronts, a CU two
+// workgroups of 256, four of 128 or eight of 64.
+//  - N <= CUs: a CU each, and its whole LDS (a step of a pile of 1500 bodies
+//    in the reference order, whose ordering and forces then fit: 14.1 -> 5.7
+//    ms; two of 4096 bodies, coloured: 11.5 -> 11.0 ms).
+//  - N <= 2 CUs: two on a CU, half its LDS each (600 worlds of 8 bodies take
+//    1.01 ms a pair of steps with 256 lanes and 0.77 with 128; 333 of 40
+//    bodies 1.49 and 1.61).
+//  - above, 128 lanes (1500 worlds of 32 bodies: 3.25 -> 2.39 ms in the
+//    reference order, 2.61 -> 1.81 coloured), and for N > 4 CUs of small
+//    worlds 64 lanes (8192 cars 9.45 -> 3.13 ms, 3000 worlds of 16 bodies
+//    4.55 -> 2.27 ms; worlds of 32 bodies 2.39 -> 3.10 in the reference
+//    order, whose parallel phases want the lanes, but 1.81 -> 1.60 coloured).
+// In the coloured order a colour is capped at the workgroup's width: fewer
+// lanes than 256 only where no world has more bodies than lanes, so that no
+// colour (its constraints share no body) reaches the cap.  Iterating to a
+// tolerance the block sums follow the width too, and it stays 256.
+static void default_shape(BatchImpl *b) {
+  const int N = b->nworlds, cu = b->cu_count;
+  const bool ref = b->order_mode == ORDER_REFERENCE;
+  const double mean = (double)b->nb / N;
+  int most = 0;
+  for (const WorldInfo &w : b->wi) most = std::max(most, w.nb);
+  b->wg = 256;
+  if (!b->tol_on) {
+    if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64)) b->wg = 64;
+    else if (N > 2 * cu && (ref || most <= 128)) b->wg = 128;
+  }
+  b->lds = lds_share(b, N <= cu ? 1 : (b->wg == 256 ? 2 : (b->wg == 128 ? 4 : 8)));
 }
 
 template <class T>
@@ -303,6 +337,7 @@ BatchImpl *batch_create_arrays(BatchArrays &A, int order_mode) {
   }
   b->wi = A.wi;
   b->wp = A.wp;
+  default_shape(b);
   // largest worlds first for the persistent queue
   std::vector<int> order(b->nworlds);
   std::iota(order.begin(), order.end(), 0);
@@ -748,6 +783,7 @@ int batch_set_tolerance(BatchImpl *b, float tol, int max_iterations, int check_e
       }))
     return 0;
   b->tol_on = tol > 0.f;
+  if (!b->shape_set) default_shape(b);
   destroy_graph(b);
   return 1;
 }
@@ -773,6 +809,10 @@ static int set_cell_scale(BatchImpl *b, float s) {
 int batch_set_launch(BatchImpl *b, int wg, float cell_scale, int grid) {
   if (wg != 64 && wg != 128 && wg != 192 && wg != 256) return 0;
   if (!(cell_scale >= 1.0f && cell_scale <= 8.0f)) return 0;
+  if (!b->shape_set) {
+    b->lds = lds_share(b, 2);   // the pool that goes with a shape set by hand
+    b->shape_set = true;
+  }
   b->wg = wg;
   b->grid = grid;
   if (!set_cell_scale(b, cell_scale)) return 0;
@@ -783,6 +823,7 @@ int batch_set_launch(BatchImpl *b, int wg, float cell_scale, int grid) {
 int batch_set_lds(BatchImpl *b, int bytes) {
   if (bytes < 0 || bytes > b->lds_max) return 0;
   b->lds = bytes & ~255;
+  b->shape_set = true;
   destroy_graph(b);
   return 1;
 }
@@ -844,6 +885,7 @@ int batch_autotune(BatchImpl *b, int trial_steps, int flags) {
   };
   double best = 1e30;
   b->sor_split = false;
+  if (!b->shape_set) batch_set_launch(b, 256, b->cell_scale, 0);
   int bw = b->wg, bg = b->grid, bl = b->lds;
   float bs = b->cell_scale;
   const float scales[] = {1.0f, 1.5f, 2.0f};
