@@ -198,8 +198,9 @@ OD_HD inline long long od_pow2(long long n) {
 OD_HD inline long long warm_bytes(int kcap, int nj) { return od_align(24LL * kcap) + 32LL * nj; }
 
 // floats of the exact-LCP workspace of one world for islands of up to m
-// rows: the matrix and its factor (m*m each), then seven vectors of m
-OD_HD inline long long lcp_ws_floats(int m) { return 2LL * m * m + 7LL * m + 64; }
+// rows: the matrix and its factor (m*m each), ten vectors of m, the rows' J
+// and inv(M) J^T
+OD_HD inline long long lcp_ws_floats(int m) { return 2LL * m * m + 34LL * m + 64; }
 
 // bytes of the coloured solver's working set held in LDS when its rows and
 // all of the conjugate-gradient state stay in global memory: the bodies' fc,
