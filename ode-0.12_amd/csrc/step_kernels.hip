@@ -1360,157 +1360,7 @@ __device__ void sor_colored(const DevBatch &B, const Ctx &c, const WorldParams &
   sor_finish(B, c, P, cons, rows, bt, corder, nrows, nact, ngroups, nk, ncons, host_contacts);
 }
 
-// LDS bytes of the reference-order constraint ordering: 12 ints per
-// constraint, 5 per body, one per joint
-__device__ inline long long ref_order_lds_bytes(int nb, int ncons, int nj) {
-  return 4LL * (12LL * ncons + 5LL * nb + nj + 16);
-}
-
-// The reference order of constraints and rows in the LDS pool: the same
-// steps as the global-memory version in phase_step (adjacency newest attach
-// first, island walk, rows in island order, per-island RNG state and Info2
-// erp), with the constraint fields gathered into LDS by all lanes first and
-// one lane walking the islands there.  The lane writes the body visit order
-// and the island table straight to global memory (nothing reads them back
-// during the walk); all lanes then write the constraint order, row offsets,
-// erp, and m = 0 for the constraints no island reaches.
-__device__ void ref_order_lds(const DevBatch &B, const Ctx &c, WorldParams &P, Cons *cons, int nk, int ncons,
-                              int *corder, int *isl, float *erp_out, int *misc, Shared &sh) {
-  const int nb = c.W.nb, nj = ncons - nk, nt = blockDim.x;
-  int *cb1 = (int *)od_pool, *cb2 = cb1 + ncons, *cm = cb2 + ncons, *ckind = cm + ncons;
-  int *cseq = ckind + ncons;               // attach sequence, then first row
-  int *cen = cseq + ncons, *ctag = cen + ncons, *cord = ctag + ncons;
-  float *cerp = (float *)(cord + ncons);   // Info2 erp seen by the constraint
-  float *cbe = cerp + ncons;               // a ball joint's own erp
-  int *adj = (int *)(cbe + ncons);         // 2 per constraint
-  int *adjs = adj + 2 * ncons;             // nb + 1
-  int *fill = adjs + nb + 1;               // fill cursors, then body tags
-  int *tag = fill;
-  int *stack = fill + nb;
-  int *ispan = stack + nb;                 // first constraint and count per island
-  int *jord = ispan + 2 * nb;              // nj
-  int *border = corder + ncons;            // body visit order (global)
-  for (int i = threadIdx.x; i < ncons; i += nt) {
-    const Cons q = cons[i];
-    cb1[i] = q.b1; cb2[i] = q.b2; cm[i] = q.m; ckind[i] = q.kind; cseq[i] = q.seq;
-    cen[i] = q.b1 >= 0 && (B.invMass[c.W.b0 + q.b1] > 0.f || (q.b2 >= 0 && B.invMass[c.W.b0 + q.b2] > 0.f));
-    cbe[i] = q.kind == JT_BALL ? B.joints[c.W.j0 + q.src].erp : 0.f;
-    ctag[i] = 0;
-  }
-  for (int b = threadIdx.x; b <= nb; b += nt) adjs[b] = 0;
-  __syncthreads();
-  // adjacency list sizes (LDS atomics), then their prefix (block scan) and
-  // the fill cursors, all lanes
-  for (int i = threadIdx.x; i < ncons; i += nt) {
-    if (cm[i] <= 0 && ckind[i] != JT_CONTACT) continue;
-    if (cb1[i] < 0) continue;
-    atomicAdd(&adjs[cb1[i] + 1], 1);
-    if (cb2[i] >= 0) atomicAdd(&adjs[cb2[i] + 1], 1);
-  }
-  __syncthreads();
-  {
-    const int per = (nb + 1 + nt - 1) / nt, d0 = threadIdx.x * per;
-    const int d1 = d0 + per < nb + 1 ? d0 + per : nb + 1;
-    int loc = 0;
-    for (int d = d0; d < d1; d++) loc += adjs[d];
-    int tot;
-    int run = block_excl_scan(loc, tot, sh);
-    for (int d = d0; d < d1; d++) { run += adjs[d]; adjs[d] = run; }
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < nb; b += nt) fill[b] = adjs[b];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int nj2 = 0;
-    for (int i = nk; i < ncons; i++) {
-      if (cb1[i] < 0) continue;
-      int s = cseq[i], p = nj2++;
-      while (p > 0 && cseq[jord[p - 1]] > s) { jord[p] = jord[p - 1]; p--; }
-      jord[p] = i;
-    }
-    int ci = nk - 1, jj = nj2 - 1;
-    while (ci >= 0 || jj >= 0) {
-      int pick;
-      if (jj < 0) pick = ci--;
-      else if (ci < 0) pick = jord[jj--];
-      else if (cseq[ci] > cseq[jord[jj]]) pick = ci--;
-      else pick = jord[jj--];
-      if (cb1[pick] < 0) continue;
-      adj[fill[cb1[pick]]++] = pick;
-      if (cb2[pick] >= 0) adj[fill[cb2[pick]]++] = pick;
-    }
-    for (int b = 0; b < nb; b++) tag[b] = 0;
-    int nic = 0, nib = 0, nisl = 0;
-    for (int bb = nb - 1; bb >= 0; bb--) {
-      if (tag[bb]) continue;
-      tag[bb] = 1;
-      int c0 = nic;
-      border[nib++] = bb;
-      int sp = 0, b = bb;
-      while (true) {
-        for (int k = adjs[b]; k < adjs[b + 1]; k++) {
-          int qi = adj[k];
-          if (ctag[qi]) continue;
-          if (!cen[qi]) { ctag[qi] = 2; continue; }
-          ctag[qi] = 1;
-          cord[nic++] = qi;
-          int other = (cb1[qi] == b) ? cb2[qi] : cb1[qi];
-          if (other >= 0 && tag[other] <= 0) {
-            tag[other] = 1;
-            stack[sp++] = other;
-          }
-        }
-        if (sp == 0) break;
-        b = stack[--sp];
-        border[nib++] = b;
-      }
-      ispan[2 * nisl + 0] = c0;
-      ispan[2 * nisl + 1] = nic - c0;
-      nisl++;
-    }
-    unsigned seed = P.seed;
-    unsigned long long shuffles = (unsigned long long)((P.iterations + 7) / 8);
-    int r = 0;
-    for (int k = 0; k < nisl; k++) {
-      int c0 = ispan[2 * k], cn = ispan[2 * k + 1];
-      int r0 = r;
-      float erp = P.erp;
-      for (int x = 0; x < cn; x++) {
-        const int i = cord[c0 + x];
-        cseq[i] = r;
-        r += cm[i];
-        if (ckind[i] == JT_BALL) erp = cbe[i];
-        cerp[i] = erp;
-      }
-      int m = r - r0;
-      isl[5 * k + 0] = c0;
-      isl[5 * k + 1] = cn;
-      isl[5 * k + 2] = r0;
-      isl[5 * k + 3] = m;
-      isl[5 * k + 4] = (int)seed;
-      if (m > 0 && m - 1 > 0) seed = lcg_skip(seed, shuffles * (unsigned long long)(m - 1));
-    }
-    P.seed = seed;
-    misc[0] = r;
-    misc[1] = nisl;
-    misc[2] = nic;
-    misc[3] = nib;
-    sh.ival[5] = nic;
-  }
-  __syncthreads();
-  const int nic = sh.ival[5];
-  for (int i = threadIdx.x; i < ncons; i += nt) {
-    if (ctag[i] != 1) {
-      cons[i].m = 0;
-    } else {
-      cons[i].row0 = cseq[i];
-      erp_out[i] = cerp[i];
-    }
-  }
-  for (int x = threadIdx.x; x < nic; x += nt) corder[x] = cord[x];
-  __syncthreads();
-}
-
+#include "ref_order.hpp"
 #include "lcp_exact.hpp"
 
 // STAGE 0: the whole step; 1: up to the coloured solver's set-up (the sweeps
@@ -1609,8 +1459,9 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
   __syncthreads();
   c.clk.lap(PH_BODIES);
   // --- constraint order, row offsets, groups
-  if (ref && ref_order_lds_bytes(nb, ncons, nj) <= B.lds_bytes) {
-    ref_order_lds(B, c, P, cons, nk, ncons, corder, isl, (float *)(color + nb), misc, sh);
+  if (ref && nb < 65535 && ncons < 65535 && ref_order_lds_bytes(nb, ncons) <= B.lds_bytes) {
+    ref_order_lds(cons, B.joints + c.W.j0, B.invMass + c.W.b0, &P, nb, nk, ncons, in.from_host, corder, isl,
+                  (float *)(color + nb), misc, (LdsChar *)od_pool, sh);
     nrows = misc[0];
     ngroups = misc[1];
   } else if (ref) {
