@@ -114,32 +114,49 @@ __device__ inline int block_sum(int v, Shared &sh) {
   return t;
 }
 
-// ascending bitonic sort of n (power of two) u64 keys; in LDS when it fits
-__device__ inline void bitonic_sort(unsigned long long *a, int n, Shared &sh, int lds_bytes) {
-  bool lds = (long long)n * 8 <= lds_bytes;
-  unsigned long long *pool = (unsigned long long *)od_pool;
-  unsigned long long *k = lds ? pool : a;
-  if (lds) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) pool[i] = a[i];
-    __syncthreads();
-  }
+// Ascending bitonic sort of n (power of two) u64 keys; in LDS when it fits.
+// A stage is bound by the latency of its compare-exchanges, so a lane takes
+// four pairs at a time, their loads before their stores, and every lane of a
+// stage has a pair (a walk over all n keys leaves half of them idle).
+__device__ inline void bitonic_stages(unsigned long long *k, int n) {
+  const int nt = blockDim.x, half = n >> 1;
   for (int size = 2; size <= n; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        int j = i ^ stride;
-        if (j > i) {
-          bool asc = (i & size) == 0;
-          unsigned long long x = k[i], y = k[j];
-          if ((x > y) == asc) { k[i] = y; k[j] = x; }
+      for (int p0 = threadIdx.x; p0 < half; p0 += 4 * nt) {
+        int lo[4];
+        unsigned long long x[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int p = min(p0 + u * nt, half - 1);
+          lo[u] = 2 * p - (p & (stride - 1));
+          x[u] = k[lo[u]];
+          y[u] = k[lo[u] + stride];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const bool asc = (lo[u] & size) == 0;
+          if (p0 + u * nt < half && (x[u] > y[u]) == asc) {
+            k[lo[u]] = y[u];
+            k[lo[u] + stride] = x[u];
+          }
         }
       }
       __syncthreads();
     }
   }
-  if (lds) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = pool[i];
-    __syncthreads();
+}
+
+__device__ inline void bitonic_sort(unsigned long long *a, int n, Shared &sh, int lds_bytes) {
+  if ((long long)n * 8 > lds_bytes) {
+    bitonic_stages(a, n);
+    return;
   }
+  unsigned long long *pool = (unsigned long long *)od_pool;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) pool[i] = a[i];
+  __syncthreads();
+  bitonic_stages(pool, n);
+  for (int i = threadIdx.x; i < n; i += blockDim.x) a[i] = pool[i];
+  __syncthreads();
 }
 
 // LDS bytes the block radix sort needs for a workgroup of nt lanes: digit
