@@ -95,8 +95,10 @@ int tape_begin(BatchImpl *b, int max_steps) {
     return 0;
   }
   t.ctrl_on.assign(max_steps, 0);
-  t.ckpt.emplace_back(new Snapshot());
-  if (!snapshot(b, *t.ckpt.back(), true)) return 0;
+  if (!t.keep) {   // (kept steps are never replayed)
+    t.ckpt.emplace_back(new Snapshot());
+    if (!snapshot(b, *t.ckpt.back(), true)) return 0;
+  }
   // the mode is latched only once every buffer it needs exists; the backward
   // pass follows the latched mode, whatever dBatchTapeKeepSteps says later
   t.kept = t.keep;
@@ -122,6 +124,8 @@ int tape_keep_steps(BatchImpl *b, bool on) {
     t.kovf.release();
     t.kcon_off.release();
     t.kjnt.release();
+    for (DevBuf *d : {&t.back.seg_st, &t.back.seg_con, &t.back.seg_nk, &t.back.seg_jnt, &t.back.gbuf, &t.back.scr})
+      d->release();
     if (t.kept) {
       t.kept = false;
       t.nsteps = 0;
@@ -171,7 +175,7 @@ int tape_step(BatchImpl *b, bool sync) {
     return 0;
   }
   t.nsteps++;
-  if (t.nsteps % t.interval == 0 && t.nsteps < t.max_steps) {
+  if (!t.kept && t.nsteps % t.interval == 0 && t.nsteps < t.max_steps) {
     t.ckpt.emplace_back(new Snapshot());
     if (!snapshot(b, *t.ckpt.back(), true)) return 0;
   }
@@ -182,7 +186,7 @@ int tape_step(BatchImpl *b, bool sync) {
 int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_in, float *grad_mu,
                   float *grad_bounce) {
   Tape &t = b->tape;
-  if (nsteps <= 0 || nsteps > t.nsteps || t.ckpt.empty()) {
+  if (nsteps <= 0 || nsteps > t.nsteps || (!t.kept && t.ckpt.empty())) {
     report_error("dBatchStepBackward: %d steps requested, %d recorded", nsteps, t.nsteps);
     return 0;
   }
@@ -191,56 +195,56 @@ int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_i
     return 0;
   }
   const int nb = b->nb, nw = b->nworlds, K = t.interval;
-  // per-world offsets of contacts and adjoint scratch
-  std::vector<long long> con_off(nw), scr_off(nw);
-  long long ncon = 0, nscr = 0;
-  for (int w = 0; w < nw; w++) {
-    con_off[w] = ncon;
-    scr_off[w] = nscr;
-    ncon += b->wi[w].kcap;
-    nscr += adj::adj_scratch_elems<float>(b->wi[w].nb, b->wi[w].kcap, b->wi[w].nj);
-    nscr = (nscr + 63) & ~63LL;
+  Tape::Back &k = t.back;
+  if (!k.nscr) {
+    // per-world offsets of contacts and adjoint scratch
+    std::vector<long long> con_off(nw), scr_off(nw);
+    long long ncon = 0, nscr = 0;
+    for (int w = 0; w < nw; w++) {
+      con_off[w] = ncon;
+      scr_off[w] = nscr;
+      ncon += b->wi[w].kcap;
+      nscr += adj::adj_scratch_elems<float>(b->wi[w].nb, b->wi[w].kcap, b->wi[w].nj);
+      nscr = (nscr + 63) & ~63LL;
+    }
+    if (!k.con_off.alloc(sizeof(long long) * nw) || !k.scr_off.alloc(sizeof(long long) * nw)) {
+      report_error("dBatchStepBackward: device allocation failed (offsets of %d worlds)", nw);
+      return 0;
+    }
+    OD_HIP(hipMemcpy(k.con_off.p, con_off.data(), sizeof(long long) * nw, hipMemcpyHostToDevice));
+    OD_HIP(hipMemcpy(k.scr_off.p, scr_off.data(), sizeof(long long) * nw, hipMemcpyHostToDevice));
+    k.ncon = ncon;
+    k.nscr = nscr;
   }
-  DevBuf d_con_off, d_scr_off, seg_st, seg_con, seg_nk, seg_jnt, gbuf, scr, gmu, gbn, stats, ctrl_save;
+  DevBuf &d_con_off = k.con_off, &d_scr_off = k.scr_off, &seg_st = k.seg_st, &seg_con = k.seg_con, &seg_nk = k.seg_nk,
+         &seg_jnt = k.seg_jnt, &gbuf = k.gbuf, &scr = k.scr, &stats = k.stats, &ctrl_save = k.ctrl_save;
+  const long long ncon = k.ncon, nscr = k.nscr;
   const size_t stbytes = sizeof(float4) * (size_t)nb;
-  bool ok = d_con_off.alloc(sizeof(long long) * nw) && d_scr_off.alloc(sizeof(long long) * nw) &&
-            seg_st.alloc(4 * stbytes * K) && seg_con.alloc(sizeof(adj::TapeContact<float>) * (size_t)ncon * K) &&
-            seg_nk.alloc(sizeof(int) * (size_t)nw * K) && gbuf.alloc(8 * stbytes) &&
-            scr.alloc(sizeof(float) * (size_t)nscr) && gmu.alloc(sizeof(float) * nw) &&
-            gbn.alloc(sizeof(float) * nw) && stats.alloc(sizeof(int) * (2 * (size_t)nw + 1)) &&
-            (b->nj == 0 || t.kept ||
-             (seg_jnt.alloc(sizeof(adj::TapeJoint<float>) * (size_t)b->nj * K) &&
-              ctrl_save.alloc(sizeof(float4) * (size_t)b->nj)));
+  // par: the per-world parameter adjoints (mu, then bounce)
+  bool ok = gbuf.alloc(8 * stbytes) && scr.alloc(sizeof(float) * (size_t)nscr) && k.par.alloc(2 * sizeof(float) * nw) &&
+            stats.alloc(sizeof(int) * (2 * (size_t)nw + 1)) &&
+            (t.kept ||
+             (seg_st.alloc(4 * stbytes * K) && seg_con.alloc(sizeof(adj::TapeContact<float>) * (size_t)ncon * K) &&
+              seg_nk.alloc(sizeof(int) * (size_t)nw * K) &&
+              (b->nj == 0 || (seg_jnt.alloc(sizeof(adj::TapeJoint<float>) * (size_t)b->nj * K) &&
+                              ctrl_save.alloc(sizeof(float4) * (size_t)b->nj)))));
   if (!ok) {
     report_error("dBatchStepBackward: device allocation failed (%lld contacts, %lld scratch floats per step)", ncon,
                  nscr);
     return 0;
   }
-  OD_HIP(hipMemcpy(d_con_off.p, con_off.data(), sizeof(long long) * nw, hipMemcpyHostToDevice));
-  OD_HIP(hipMemcpy(d_scr_off.p, scr_off.data(), sizeof(long long) * nw, hipMemcpyHostToDevice));
-  OD_HIP(hipMemset(gmu.p, 0, gmu.n));
-  OD_HIP(hipMemset(gbn.p, 0, gbn.n));
-  OD_HIP(hipMemset(stats.p, 0, stats.n));
+  float *const gmu = k.par.as<float>(), *const gbn = gmu + nw;
+  OD_HIP(hipMemsetAsync(gmu, 0, 2 * sizeof(float) * nw, b->stream));
+  OD_HIP(hipMemsetAsync(stats.p, 0, sizeof(int) * (2 * (size_t)nw + 1), b->stream));
   // adjoint buffers: two sets of (x, q, v, w) float4 arrays
   float4 *G[2][4];
   for (int s = 0; s < 2; s++)
-    for (int k = 0; k < 4; k++) G[s][k] = gbuf.as<float4>() + (size_t)(4 * s + k) * nb;
-  {
-    std::vector<float4> h[4];
-    for (int k = 0; k < 4; k++) h[k].assign(nb, make_float4(0, 0, 0, 0));
-    for (int i = 0; i < nb; i++) {
-      const float *g = grad_out + 13 * (size_t)i;
-      h[0][i] = make_float4(g[0], g[1], g[2], 0);
-      h[1][i] = make_float4(g[3], g[4], g[5], g[6]);
-      h[2][i] = make_float4(g[7], g[8], g[9], 0);
-      h[3][i] = make_float4(g[10], g[11], g[12], 0);
-    }
-    for (int k = 0; k < 4; k++) OD_HIP(hipMemcpy(G[0][k], h[k].data(), stbytes, hipMemcpyHostToDevice));
-  }
+    for (int j = 0; j < 4; j++) G[s][j] = gbuf.as<float4>() + (size_t)(4 * s + j) * nb;
+  if (!state_in(b, grad_out, G[0], nullptr)) return 0;
   int cur = 0;
-  // the state at the end of the tape, restored afterwards
-  Snapshot endsnap;
-  if (!snapshot(b, endsnap, true)) return 0;
+  // the state at the end of the tape, restored after the replays
+  Snapshot &endsnap = k.end;
+  if (!t.kept && !snapshot(b, endsnap, true)) return 0;
   const int T = t.nsteps, first = T - nsteps;
   bool fail = false;
   if (t.kept) {
@@ -259,7 +263,7 @@ int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_i
       float4 *gout[4] = {G[1 - cur][0], G[1 - cur][1], G[1 - cur][2], G[1 - cur][3]};
       OD_HIP(launch_adjoint_step(b->dev, st4, t.kcon.as<adj::TapeContact<float>>() + (size_t)s * t.kncon,
                                  t.kcon_off.as<long long>(), t.knk.as<int>() + (size_t)s * nw, gin, gout,
-                                 gmu.as<float>(), gbn.as<float>(), stats.as<int>(), scr.as<float>(),
+                                 gmu, gbn, stats.as<int>(), scr.as<float>(),
                                  d_scr_off.as<long long>(), t.act_tol, t.lin_tol, t.lin_maxit, 256,
                                  b->nj ? t.kjnt.as<adj::TapeJoint<float>>() + (size_t)s * b->nj : nullptr,
                                  b->stream));
@@ -327,7 +331,7 @@ int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_i
       float4 *gout[4] = {G[1 - cur][0], G[1 - cur][1], G[1 - cur][2], G[1 - cur][3]};
       OD_HIP(launch_adjoint_step(b->dev, st4, seg_con.as<adj::TapeContact<float>>() + (size_t)j * ncon,
                                  d_con_off.as<long long>(), seg_nk.as<int>() + (size_t)j * nw, gin, gout,
-                                 gmu.as<float>(), gbn.as<float>(), stats.as<int>(), scr.as<float>(),
+                                 gmu, gbn, stats.as<int>(), scr.as<float>(),
                                  d_scr_off.as<long long>(), t.act_tol, t.lin_tol, t.lin_maxit, 256,
                                  b->nj ? seg_jnt.as<adj::TapeJoint<float>>() + (size_t)j * b->nj : nullptr,
                                  b->stream));
@@ -339,25 +343,11 @@ int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_i
     OD_HIP(hipMemcpyAsync(b->d.ctrl.p, ctrl_save.p, sizeof(float4) * b->nj, hipMemcpyDeviceToDevice, b->stream));
     ctrl_restore.armed = false;
   }
-  if (!snapshot(b, endsnap, false)) return 0;
+  if (!t.kept && !snapshot(b, endsnap, false)) return 0;
   if (fail) return 0;
-  OD_HIP(hipStreamSynchronize(b->stream));
-  {
-    std::vector<float4> h[4];
-    for (int k = 0; k < 4; k++) {
-      h[k].resize(nb);
-      OD_HIP(hipMemcpy(h[k].data(), G[cur][k], stbytes, hipMemcpyDeviceToHost));
-    }
-    for (int i = 0; i < nb; i++) {
-      float *g = grad_in + 13 * (size_t)i;
-      g[0] = h[0][i].x; g[1] = h[0][i].y; g[2] = h[0][i].z;
-      g[3] = h[1][i].x; g[4] = h[1][i].y; g[5] = h[1][i].z; g[6] = h[1][i].w;
-      g[7] = h[2][i].x; g[8] = h[2][i].y; g[9] = h[2][i].z;
-      g[10] = h[3][i].x; g[11] = h[3][i].y; g[12] = h[3][i].z;
-    }
-  }
-  if (grad_mu) OD_HIP(hipMemcpy(grad_mu, gmu.p, sizeof(float) * nw, hipMemcpyDeviceToHost));
-  if (grad_bounce) OD_HIP(hipMemcpy(grad_bounce, gbn.p, sizeof(float) * nw, hipMemcpyDeviceToHost));
+  if (!state_out(b, G[cur], grad_in)) return 0;
+  if (grad_mu) OD_HIP(hipMemcpy(grad_mu, gmu, sizeof(float) * nw, hipMemcpyDeviceToHost));
+  if (grad_bounce) OD_HIP(hipMemcpy(grad_bounce, gbn, sizeof(float) * nw, hipMemcpyDeviceToHost));
   std::vector<int> st(2 * (size_t)nw);
   OD_HIP(hipMemcpy(st.data(), stats.p, sizeof(int) * st.size(), hipMemcpyDeviceToHost));
   t.iters = 0;

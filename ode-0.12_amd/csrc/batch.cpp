@@ -359,7 +359,9 @@ BatchImpl *batch_create_arrays(BatchArrays &A, int order_mode) {
             d.residual.alloc(sizeof(float) * (size_t)b->nworlds) && d.work_counter.alloc(64 * WORK_QUEUES) &&
             d.scratch.alloc((size_t)scratch) && d.warm.alloc((size_t)(warm > 0 ? warm : 256)) &&
             d.warm_n.alloc(sizeof(int) * (size_t)b->nworlds) && d.ctrl.alloc(sizeof(float4) * (size_t)(nj ? nj : 1)) &&
-            d.prof.alloc(sizeof(unsigned long long) * PH_N * (size_t)b->nworlds);
+            d.prof.alloc(sizeof(unsigned long long) * PH_N * (size_t)b->nworlds) &&
+            (sizeof(float) * 13 * (size_t)nb <= XFER_PINNED ? d.xfer.alloc(sizeof(float) * 13 * (size_t)nb)
+                                                            : d.xfer_dev.alloc(sizeof(float) * 13 * (size_t)nb));
   if (!ok) {
     report_error("batch setup failed (%lld scratch bytes)", scratch);
     batch_destroy(b);
@@ -614,51 +616,44 @@ int batch_launch_once(BatchImpl *b) {
   return 1;
 }
 
-int batch_get_state(BatchImpl *b, float *out) {
+int state_out(BatchImpl *b, const float4 *const a[4], float *out) {
+  const size_t bytes = sizeof(float) * 13 * (size_t)b->nb;
+  if (b->d.xfer.p) {
+    OD_HIP(launch_pack_state(a, b->nb, b->d.xfer.as<float>(), b->stream));
+    OD_HIP(hipStreamSynchronize(b->stream));
+    std::memcpy(out, b->d.xfer.p, bytes);
+    return 1;
+  }
+  OD_HIP(launch_pack_state(a, b->nb, b->d.xfer_dev.as<float>(), b->stream));
+  OD_HIP(hipMemcpyAsync(out, b->d.xfer_dev.p, bytes, hipMemcpyDeviceToHost, b->stream));
   OD_HIP(hipStreamSynchronize(b->stream));
-  std::vector<float4> p(b->nb), q(b->nb), v(b->nb), w(b->nb);
-  if (b->nb) {
-    OD_HIP(hipMemcpy(p.data(), b->d.pos.p, sizeof(float4) * b->nb, hipMemcpyDeviceToHost));
-    OD_HIP(hipMemcpy(q.data(), b->d.q.p, sizeof(float4) * b->nb, hipMemcpyDeviceToHost));
-    OD_HIP(hipMemcpy(v.data(), b->d.lvel.p, sizeof(float4) * b->nb, hipMemcpyDeviceToHost));
-    OD_HIP(hipMemcpy(w.data(), b->d.avel.p, sizeof(float4) * b->nb, hipMemcpyDeviceToHost));
-  }
-  for (int i = 0; i < b->nb; i++) {
-    float *r = out + 13 * (size_t)i;
-    r[0] = p[i].x; r[1] = p[i].y; r[2] = p[i].z;
-    r[3] = q[i].x; r[4] = q[i].y; r[5] = q[i].z; r[6] = q[i].w;
-    r[7] = v[i].x; r[8] = v[i].y; r[9] = v[i].z;
-    r[10] = w[i].x; r[11] = w[i].y; r[12] = w[i].z;
-  }
   return 1;
 }
 
-template <class F>
-static int patch_params(BatchImpl *b, F f);
+int state_in(BatchImpl *b, const float *in, float4 *const a[4], float4 *R) {
+  const size_t bytes = sizeof(float) * 13 * (size_t)b->nb;
+  OD_HIP(hipStreamSynchronize(b->stream));
+  if (b->d.xfer.p) std::memcpy(b->d.xfer.p, in, bytes);
+  else OD_HIP(hipMemcpy(b->d.xfer_dev.p, in, bytes, hipMemcpyHostToDevice));
+  OD_HIP(launch_unpack_state(b->d.xfer.p ? b->d.xfer.as<float>() : b->d.xfer_dev.as<float>(), b->nb, a, R, b->stream));
+  return 1;
+}
+
+int batch_get_state(BatchImpl *b, float *out) {
+  const float4 *st[4] = {b->d.pos.as<float4>(), b->d.q.as<float4>(), b->d.lvel.as<float4>(), b->d.avel.as<float4>()};
+  return state_out(b, st, out);
+}
 
 int batch_set_state(BatchImpl *b, const float *in) {
-  OD_HIP(hipStreamSynchronize(b->stream));
-  std::vector<float4> p(b->nb), q(b->nb), v(b->nb), w(b->nb);
-  for (int i = 0; i < b->nb; i++) {
-    const float *r = in + 13 * (size_t)i;
-    p[i] = make_float4(r[0], r[1], r[2], 0);
-    q[i] = make_float4(r[3], r[4], r[5], r[6]);
-    v[i] = make_float4(r[7], r[8], r[9], 0);
-    w[i] = make_float4(r[10], r[11], r[12], 0);
-  }
-  if (b->nb) {
-    OD_HIP(hipMemcpy(b->d.pos.p, p.data(), sizeof(float4) * b->nb, hipMemcpyHostToDevice));
-    OD_HIP(hipMemcpy(b->d.q.p, q.data(), sizeof(float4) * b->nb, hipMemcpyHostToDevice));
-    OD_HIP(hipMemcpy(b->d.lvel.p, v.data(), sizeof(float4) * b->nb, hipMemcpyHostToDevice));
-    OD_HIP(hipMemcpy(b->d.avel.p, w.data(), sizeof(float4) * b->nb, hipMemcpyHostToDevice));
-  }
-  // the previous impulses belong to the old state: the next solve starts from zero
-  OD_HIP(hipMemset(b->d.warm_n.p, 0xff, b->d.warm_n.n));
   refresh_dev(b);
-  if (launch_init_rot(b->dev, b->nb, b->stream) != hipSuccess) return 0;
+  float4 *st[4] = {b->d.pos.as<float4>(), b->d.q.as<float4>(), b->d.lvel.as<float4>(), b->d.avel.as<float4>()};
+  if (!state_in(b, in, st, b->d.R.as<float4>())) return 0;
+  // a new state revives frozen worlds; the previous impulses belong to the
+  // old one
+  for (auto &p : b->wp) p.dead = 0;
+  OD_HIP(launch_revive(b->d.wp.as<WorldParams>(), b->d.warm_n.as<int>(), b->nworlds, b->stream));
   OD_HIP(hipStreamSynchronize(b->stream));
-  // a new state revives frozen worlds
-  return patch_params(b, [](WorldParams &p) { p.dead = 0; });
+  return 1;
 }
 
 int batch_counters(BatchImpl *b, long long *out5) {

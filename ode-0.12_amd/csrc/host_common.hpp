@@ -50,6 +50,30 @@ struct DevBuf {
   template <class T> T *as() const { return (T *)p; }
 };
 
+// Pinned host memory that kernels read and write directly.
+struct HostBuf {
+  void *p = nullptr;
+  size_t n = 0;
+  HostBuf() = default;
+  HostBuf(const HostBuf &) = delete;
+  HostBuf &operator=(const HostBuf &) = delete;
+  ~HostBuf() { release(); }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  bool alloc(size_t bytes) {
+    if (bytes <= n && p) return true;
+    release();
+    if (bytes == 0) bytes = 16;
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) { p = nullptr; return false; }
+    n = bytes;
+    return true;
+  }
+  template <class T> T *as() const { return (T *)p; }
+};
+
 // ---------------------------------------------------------------- setup math
 // (host copies of the reference's setters; float, 3x4 row-major rotations)
 
@@ -276,6 +300,11 @@ enum {
 hipError_t launch_world_kernel(int mode, const DevBatch &B, int first_world, int nworlds_launch, int grid, int wg,
                                int api_maxc, hipStream_t st, int queue = 0);
 hipError_t launch_init_rot(const DevBatch &B, int nbodies, hipStream_t st);
+// 13 floats per body from / into pos, q, lvel, avel (state_kernels.hip)
+hipError_t launch_pack_state(const float4 *const a[4], int n, float *out, hipStream_t st);
+hipError_t launch_unpack_state(const float *in, int n, float4 *const a[4], float4 *R, hipStream_t st);
+hipError_t launch_revive(WorldParams *wp, int *warm_n, int nworlds, hipStream_t st);
+hipError_t launch_api_gather(const DevBatch &B, int nb, int ng, int *out, hipStream_t st);
 // the persistent queue's order of B.world_order by expected cost (rank: the
 // static order; est: the per-world cost estimates it keeps); at most 8192
 // worlds

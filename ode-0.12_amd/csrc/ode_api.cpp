@@ -61,7 +61,12 @@ struct dxWorld {
   bool struct_dirty = true, state_dirty = true, joints_dirty = true, rank_dirty = true;
   bool device_newer = false;
   bool tape = false;
-  DevBuf cin, cin_start, cin_count, feedback, pairs_out, pcount_out, contacts_out, one_out, one_n;
+  DevBuf cin;                              // first contact (0) and count, 64 bytes on the contacts
+  // written by the kernels, read by the host without a copy
+  HostBuf collide_out;                     // counters, pairs, contact counts, contacts (dSpaceCollide)
+  HostBuf step_out;                        // what a step hands back (api_gather_kernel)
+  std::vector<float> stepped;              // the state of the last step, if the device's is the newer one
+  DevBuf feedback, one_out, one_n;
   // the last dWorldQuickStep recorded for dWorldQuickStepBackward: pre-step
   // state (pos, q, lvel, avel; nb float4 each), contacts with impulses, and
   // the contact policy the adjoint differentiates
@@ -205,12 +210,21 @@ void geom_detach_body(dxGeom *g) {
   g->body = nullptr;
 }
 
+// dSpaceCollide's outputs in one block: counters (64 bytes), pairs, contacts
+// per pair, contacts
+size_t collide_out_counts(int pcap) { return 64 + sizeof(PairRec) * (size_t)pcap; }
+size_t collide_out_contacts(int pcap) { return (collide_out_counts(pcap) + sizeof(int) * ((size_t)pcap + 1) + 63) & ~(size_t)63; }
+
 // device state -> host copies
 int pull_state(dxWorld *w) {
   if (!w->device_newer || !w->mir) return 1;
   BatchImpl *m = w->mir;
-  std::vector<float> st(13 * (size_t)m->nb);
-  if (!batch_get_state(m, st.data())) return 0;
+  std::vector<float> st;
+  st.swap(w->stepped);
+  if (st.size() != 13 * (size_t)m->nb) {
+    st.resize(13 * (size_t)m->nb);
+    if (!batch_get_state(m, st.data())) return 0;
+  }
   for (dxBody *b : w->bodies) {
     if (b->mindex < 0) continue;
     const float *r = &st[13 * (size_t)b->mindex];
@@ -311,9 +325,9 @@ int build_mirror(dxWorld *w, dxSpace *sp) {
   w->mir_space = sp;
   w->pcap = wi.pcap;
   w->kcap = wi.kcap;
-  if (!w->pairs_out.alloc(sizeof(PairRec) * wi.pcap) || !w->pcount_out.alloc(sizeof(int) * (wi.pcap + 1)) ||
-      !w->contacts_out.alloc(sizeof(ContactRec) * wi.kcap) || !w->cin_start.alloc(sizeof(int)) ||
-      !w->cin_count.alloc(sizeof(int)) || !w->one_out.alloc(sizeof(CPoint) * MAX_SLOTS) || !w->one_n.alloc(16)) {
+  if (!w->collide_out.alloc(collide_out_contacts(wi.pcap) + sizeof(ContactRec) * wi.kcap) ||
+      !w->step_out.alloc(sizeof(int) * (CNT_N + 1 + w->mgeoms.size() + 13 * (size_t)w->mir->nb)) ||
+      !w->one_out.alloc(sizeof(CPoint) * MAX_SLOTS) || !w->one_n.alloc(16)) {
     report_error("device allocation failed");
     return 0;
   }
@@ -367,8 +381,7 @@ int sync_mirror(dxWorld *w, dxSpace *sp) {
 
 int world_params_upload(dxWorld *w, float dt, int maxc, int exact) {
   BatchImpl *m = w->mir;
-  WorldParams P;
-  OD_HIP(hipMemcpy(&P, m->d.wp.p, sizeof(P), hipMemcpyDeviceToHost));
+  WorldParams P = m->wp[0];   // the device's differs in the generator state (set below) and `dead` (the batch's)
   for (int k = 0; k < 3; k++) P.gravity[k] = w->gravity[k];
   P.erp = w->erp; P.cfm = w->cfm; P.iterations = w->iterations; P.sor_w = w->sor_w;
   P.max_vel = w->max_vel; P.min_depth = w->min_depth;
@@ -377,6 +390,7 @@ int world_params_upload(dxWorld *w, float dt, int maxc, int exact) {
   P.seed = (unsigned)global_seed();
   if (w->mir_space) { P.hash_min = w->mir_space->minlevel; P.hash_max = w->mir_space->maxlevel; }
   P.exact = exact;
+  m->wp[0] = P;
   OD_HIP(hipMemcpy(m->d.wp.p, &P, sizeof(P), hipMemcpyHostToDevice));
   return 1;
 }
@@ -586,11 +600,15 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
     if (!J.empty()) OD_HIP(hipMemcpy(m->d.joints.p, J.data(), sizeof(JointDev) * J.size(), hipMemcpyHostToDevice));
     w->joints_dirty = false;
   }
-  if (!w->cin.alloc(sizeof(ContactIn) * (cin.size() + 1))) return 0;
-  if (!cin.empty()) OD_HIP(hipMemcpy(w->cin.p, cin.data(), sizeof(ContactIn) * cin.size(), hipMemcpyHostToDevice));
-  int zero = 0, nk = (int)cin.size();
-  OD_HIP(hipMemcpy(w->cin_start.p, &zero, sizeof(int), hipMemcpyHostToDevice));
-  OD_HIP(hipMemcpy(w->cin_count.p, &nk, sizeof(int), hipMemcpyHostToDevice));
+  const int nk = (int)cin.size();
+  if (!w->cin.alloc(64 + sizeof(ContactIn) * (cin.size() + 1))) return 0;
+  {
+    std::vector<char> up(64 + sizeof(ContactIn) * cin.size(), 0);
+    std::memcpy(up.data() + sizeof(int), &nk, sizeof(int));
+    if (nk) std::memcpy(up.data() + 64, cin.data(), sizeof(ContactIn) * cin.size());
+    OD_HIP(hipMemcpy(w->cin.p, up.data(), up.size(), hipMemcpyHostToDevice));
+  }
+  const ContactIn *dcin = (const ContactIn *)(w->cin.as<char>() + 64);
   if (!w->feedback.alloc(sizeof(float) * 12 * (fbs.size() + 1))) return 0;
   if (!fbs.empty()) {
     // the user's current values: the kernel overwrites what the reference
@@ -607,9 +625,9 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
   if (!world_params_upload(w, stepsize, 0, exact ? 1 : 0)) return 0;
   refresh_dev(m);
   DevBatch D = m->dev;
-  D.cin = w->cin.as<ContactIn>();
-  D.cin_start = w->cin_start.as<int>();
-  D.cin_count = w->cin_count.as<int>();
+  D.cin = dcin;
+  D.cin_start = w->cin.as<int>();
+  D.cin_count = w->cin.as<int>() + 1;
   D.feedback = fbs.empty() ? nullptr : w->feedback.as<float>();
   D.ctrl = nullptr;
   if (exact) {
@@ -639,15 +657,19 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
   }
   OD_HIP(launch_world_kernel(KM_API_STEP, D, 0, 1, 0, m->wg, 0, m->stream));
   if (record)
-    OD_HIP(launch_api_tape_capture(D, w->cin.as<ContactIn>(), nk, w->tape_con.as<adj::TapeContact<float>>(),
+    OD_HIP(launch_api_tape_capture(D, dcin, nk, w->tape_con.as<adj::TapeContact<float>>(),
                                    w->tape_nk.as<int>(), m->nj ? w->tape_jnt.as<adj::TapeJoint<float>>() : nullptr,
                                    m->stream));
+  // counters, generator state, space order and state
+  const size_t ng = w->mgeoms.size();
+  OD_HIP(launch_api_gather(D, m->nb, (int)ng, w->step_out.as<int>(), m->stream));
   OD_HIP(hipStreamSynchronize(m->stream));
-  long long cnt[5];
-  batch_counters(m, cnt);
-  if (cnt[4]) {
-    report_error("%s: %s (flags %lld)", who,
-                 (cnt[4] & OVF_LCP) ? "the LCP solve did not finish" : "device capacity exceeded", cnt[4]);
+  const int *out = w->step_out.as<int>();
+  const int ovf = out[CNT_OVERFLOW];
+  w->stepped.clear();
+  if (ovf) {
+    report_error("%s: %s (flags %d)", who,
+                 (ovf & OVF_LCP) ? "the LCP solve did not finish" : "device capacity exceeded", ovf);
     return 0;
   }
   if (!exact) w->tape_ok = record;
@@ -661,9 +683,7 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
     }
   }
   // RNG state, feedback, joint limit state, space order
-  WorldParams P;
-  OD_HIP(hipMemcpy(&P, m->d.wp.p, sizeof(P), hipMemcpyDeviceToHost));
-  global_seed() = P.seed;
+  global_seed() = (unsigned)out[CNT_N];
   if (!fbs.empty()) {
     std::vector<float> f(12 * fbs.size());
     OD_HIP(hipMemcpy(f.data(), w->feedback.p, sizeof(float) * f.size(), hipMemcpyDeviceToHost));
@@ -684,10 +704,9 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
     }
   }
   if (w->mir_space && !w->mgeoms.empty()) {
-    std::vector<int> rk(w->mgeoms.size());
-    OD_HIP(hipMemcpy(rk.data(), m->d.grank.p, sizeof(int) * rk.size(), hipMemcpyDeviceToHost));
-    std::vector<dxGeom *> L(rk.size());
-    for (size_t g = 0; g < rk.size(); g++) L[rk[g]] = w->mgeoms[g];
+    const int *rk = out + CNT_N + 1;
+    std::vector<dxGeom *> L(ng);
+    for (size_t g = 0; g < ng; g++) L[rk[g]] = w->mgeoms[g];
     w->mir_space->list = L;
     for (dxGeom *g : w->mgeoms)
       if (g->body) g->dirty = true;
@@ -695,6 +714,8 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
   for (dxBody *b : w->bodies) {
     for (int k = 0; k < 3; k++) { b->facc[k] = 0; b->tacc[k] = 0; }
   }
+  w->stepped.resize(13 * (size_t)m->nb);
+  if (m->nb) std::memcpy(w->stepped.data(), out + CNT_N + 1 + ng, sizeof(float) * w->stepped.size());
   w->device_newer = true;
   return 1;
 }
@@ -1412,27 +1433,25 @@ void dSpaceCollide(dSpaceID s, void *data, dNearCallback *cb) {
   if (!world_params_upload(w, 0, s->cached_maxc, 0)) return;
   refresh_dev(m);
   DevBatch D = m->dev;
-  D.pairs_out = w->pairs_out.as<PairRec>();
-  D.pcount_out = w->pcount_out.as<int>();
-  D.contacts_out = w->contacts_out.as<ContactRec>();
+  const size_t o_counts = collide_out_counts(w->pcap), o_con = collide_out_contacts(w->pcap);
+  char *dout = w->collide_out.as<char>();
+  D.counters = (int *)dout;
+  D.pairs_out = (PairRec *)(dout + 64);
+  D.pcount_out = (int *)(dout + o_counts);
+  D.contacts_out = (ContactRec *)(dout + o_con);
   D.ctrl = nullptr;
   if (launch_world_kernel(KM_API_COLLIDE, D, 0, 1, 0, m->wg, s->cached_maxc, m->stream) != hipSuccess ||
       hipStreamSynchronize(m->stream) != hipSuccess) {
     report_error("dSpaceCollide: collide kernel failed");
     return;
   }
-  long long cnt[5];
-  batch_counters(m, cnt);
-  if (cnt[4]) report_error("dSpaceCollide: device capacity exceeded (flags %lld)", cnt[4]);
-  int np = (int)cnt[0], nk = (int)cnt[1];
-  std::vector<PairRec> pr(np);
-  std::vector<int> pc(np);
-  std::vector<ContactRec> cr(nk);
-  if (np) {
-    (void)hipMemcpy(pr.data(), w->pairs_out.p, sizeof(PairRec) * np, hipMemcpyDeviceToHost);
-    (void)hipMemcpy(pc.data(), w->pcount_out.p, sizeof(int) * np, hipMemcpyDeviceToHost);
-  }
-  if (nk) (void)hipMemcpy(cr.data(), w->contacts_out.p, sizeof(ContactRec) * nk, hipMemcpyDeviceToHost);
+  const int *cnt = (const int *)dout;
+  if (cnt[CNT_OVERFLOW]) report_error("dSpaceCollide: device capacity exceeded (flags %d)", cnt[CNT_OVERFLOW]);
+  const int np = cnt[CNT_PAIRS], nk = cnt[CNT_CONTACTS];
+  // (copies: a callback may collide another space of the world)
+  const std::vector<PairRec> pr((const PairRec *)(dout + 64), (const PairRec *)(dout + 64) + np);
+  const std::vector<int> pc((const int *)(dout + o_counts), (const int *)(dout + o_counts) + np);
+  const std::vector<ContactRec> cr((const ContactRec *)(dout + o_con), (const ContactRec *)(dout + o_con) + nk);
   for (dxGeom *g : s->list) g->dirty = false;
   std::vector<dxGeom *> mg = w->mgeoms;
   int off = 0;

@@ -37,7 +37,17 @@ struct Tape {
   // the joint controls each recorded step ran with (replays re-apply them)
   DevBuf kctrl;
   std::vector<char> ctrl_on;
+  // the backward pass's buffers, kept from one call to the next
+  struct Back {
+    DevBuf con_off, scr_off, seg_st, seg_con, seg_nk, seg_jnt, gbuf, scr, par, stats, ctrl_save;
+    Snapshot end;
+    long long ncon = 0, nscr = 0;   // contacts and scratch floats of all worlds (con_off and scr_off set)
+  } back;
 };
+
+// A pinned buffer saves the copy's 20 to 30 us, but a large one costs more
+// than that when it is first mapped (13.6 MB: 6 ms on the first pass).
+constexpr size_t XFER_PINNED = 1u << 20;
 
 // device arrays of a batch
 struct BatchBufs {
@@ -46,6 +56,10 @@ struct BatchBufs {
   DevBuf joints, adj_start, adj_other, bgeom_start, bgeom;
   DevBuf ctrl, counters, residual, work_counter, world_order, world_rank, cost_est, scratch, feedback, prof, warm,
       warm_n;
+  // 13 floats per body on their way between host and device: pinned memory up
+  // to XFER_PINNED bytes, else device memory
+  HostBuf xfer;
+  DevBuf xfer_dev;
 };
 
 struct BatchImpl {
@@ -106,6 +120,10 @@ void batch_destroy(BatchImpl *b);
 int batch_step(BatchImpl *b, int nsteps, bool sync);
 int batch_step_plain(BatchImpl *b, int nsteps, bool sync);
 int batch_launch_once(BatchImpl *b);
+// 13 floats per body from / into float4 arrays (pos, q, lvel, avel, or their
+// gradients), after all work on the batch's stream
+int state_out(BatchImpl *b, const float4 *const a[4], float *out);
+int state_in(BatchImpl *b, const float *in, float4 *const a[4], float4 *R);
 int batch_get_state(BatchImpl *b, float *out);
 int batch_set_state(BatchImpl *b, const float *in);
 int batch_counters(BatchImpl *b, long long *out5);
