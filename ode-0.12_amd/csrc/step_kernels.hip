@@ -1380,6 +1380,36 @@ __device__ void sor_colored(const DevBatch &B, const Ctx &c, const WorldParams &
 #include "ref_order.hpp"
 #include "lcp_exact.hpp"
 
+// inv(M) J^T, rhs, cfm and ad of a row whose rhs holds c.  t1, t2: its
+// bodies' temporaries (t2 null: one body): world inverse inertia 0..8, v/h +
+// inv(M) f_ext 15..20.
+__device__ inline void finish_row(Row &R, const float *t1, const float *t2, float im1, float im2, float hinv,
+                                  float sor_w) {
+  float s = 0.f;
+  for (int k = 0; k < 6; k++) s += R.J[k] * t1[15 + k];
+  float d = 0.f;
+  for (int k = 0; k < 3; k++) R.iMJ[k] = im1 * R.J[k];
+  for (int k = 0; k < 3; k++) R.iMJ[3 + k] = t1[3 * k] * R.J[3] + t1[3 * k + 1] * R.J[4] + t1[3 * k + 2] * R.J[5];
+  for (int k = 0; k < 6; k++) d += R.iMJ[k] * R.J[k];
+  if (t2) {
+    for (int k = 0; k < 6; k++) s += R.J[6 + k] * t2[15 + k];
+    for (int k = 0; k < 3; k++) R.iMJ[6 + k] = im2 * R.J[6 + k];
+    for (int k = 0; k < 3; k++) R.iMJ[9 + k] = t2[3 * k] * R.J[9] + t2[3 * k + 1] * R.J[10] + t2[3 * k + 2] * R.J[11];
+    for (int k = 6; k < 12; k++) d += R.iMJ[k] * R.J[k];
+  } else {
+    for (int k = 6; k < 12; k++) R.iMJ[k] = 0.f;
+  }
+  R.rhs = R.rhs * hinv - s;
+  R.cfm = R.cfm * hinv;
+  R.ad = sor_w / (d + R.cfm);
+  R.lambda = 0.f;
+}
+
+__device__ inline void store_row(Row *dst, const Row &R) {
+  static_assert(sizeof(Row) % 16 == 0, "rows are written 16 bytes at a time");
+  __builtin_memcpy(__builtin_assume_aligned(dst, 16), &R, sizeof(Row));
+}
+
 // STAGE 0: the whole step; 1: up to the coloured solver's set-up (the sweeps
 // and the rest run in later kernels); 2: after the sweeps (write-back,
 // velocities, integration)
@@ -1627,15 +1657,20 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
     __syncthreads();
     return;
   }
-  // --- getInfo2 (quickstep.cpp:764-830): one constraint per lane
+  // --- getInfo2 (quickstep.cpp:764-830) and rhs = c/h - J (v/h + inv(M)
+  //     f_ext), cfm /= h (832-857), one constraint per lane.  The joints come
+  //     first: a motor pushing against its limit adds to f_ext.  A contact's
+  //     rows are built and finished in registers and written once, 16 bytes
+  //     at a time: written word by word, read back and written again they
+  //     cost a pass of 64 cache lines per word (4096 uneven worlds: 2047 ->
+  //     1391 workgroup-ms in 4 steps).
   const float *erp_of = ref ? (const float *)(color + nb) : nullptr;
-  for (int i = threadIdx.x; i < ncons; i += blockDim.x) {
+  for (int i = nk + threadIdx.x; i < ncons; i += blockDim.x) {
     Cons &q = cons[i];
     if (q.m <= 0) continue;
     Row *r = rows + q.row0;
-    float cfm0 = P.cfm;
     for (int k = 0; k < q.m; k++) {
-      row_clear(r[k], cfm0);
+      row_clear(r[k], P.cfm);
       r[k].b1 = q.b1;
       r[k].b2 = q.b2;
     }
@@ -1643,49 +1678,23 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
     BodyPose s2;
     if (q.b2 >= 0) s2 = load_pose(B, c.W.b0 + q.b2);
     const BodyPose *p2 = q.b2 >= 0 ? &s2 : nullptr;
-    float erp = erp_of ? erp_of[i] : P.erp;
-    if (q.kind == JT_CONTACT) {
-      float3 cpos, cn;
-      float cd;
-      bool rev;
-      Surf s;
-      if (in.from_host) {
-        const ContactIn &ci = B.cin[B.cin_start[c.w] + q.src];
-        cpos = mk3(ci.pos[0], ci.pos[1], ci.pos[2]);
-        cn = mk3(ci.normal[0], ci.normal[1], ci.normal[2]);
-        cd = ci.depth;
-        rev = (ci.flags & JF_REVERSE) != 0;
-        s = host_surface(ci);
-      } else {
-        const ContactRec &cr = con[q.src];
-        cpos = mk3(cr.pos[0], cr.pos[1], cr.pos[2]);
-        cn = mk3(cr.normal[0], cr.normal[1], cr.normal[2]);
-        cd = cr.depth;
-        rev = (cr.flags & JF_REVERSE) != 0;
-        s = world_surface(P);
-      }
-      int m = contact_info1(s);
-      contact_info2(r, m, s, cpos, cn, cd, rev, s1, p2, hinv, erp, P.min_depth, P.max_vel);
-    } else {
-      JointDev &j = B.joints[c.W.j0 + q.src];
-      float3 e1 = mk3(0.f, 0.f, 0.f), e2 = mk3(0.f, 0.f, 0.f);
-      float e = erp;
-      joint_info2(j, r, s1, p2, hinv, e, e1, e2);
-      float *t1 = bt + 32 * q.b1 + 21;
-      if (e1.x != 0.f || e1.y != 0.f || e1.z != 0.f) {
-        // a motor pushing against its limit: torque applied below in order
-        atomicAdd(&t1[0], e1.x); atomicAdd(&t1[1], e1.y); atomicAdd(&t1[2], e1.z);
-        if (q.b2 >= 0) {
-          float *t2 = bt + 32 * q.b2 + 21;
-          atomicAdd(&t2[0], e2.x); atomicAdd(&t2[1], e2.y); atomicAdd(&t2[2], e2.z);
-        }
+    JointDev &j = B.joints[c.W.j0 + q.src];
+    float3 e1 = mk3(0.f, 0.f, 0.f), e2 = mk3(0.f, 0.f, 0.f);
+    float e = erp_of ? erp_of[i] : P.erp;
+    joint_info2(j, r, s1, p2, hinv, e, e1, e2);
+    float *t1 = bt + 32 * q.b1 + 21;
+    if (e1.x != 0.f || e1.y != 0.f || e1.z != 0.f) {
+      // a motor pushing against its limit: torque applied below in order
+      atomicAdd(&t1[0], e1.x); atomicAdd(&t1[1], e1.y); atomicAdd(&t1[2], e1.z);
+      if (q.b2 >= 0) {
+        float *t2 = bt + 32 * q.b2 + 21;
+        atomicAdd(&t2[0], e2.x); atomicAdd(&t2[1], e2.y); atomicAdd(&t2[2], e2.z);
       }
     }
     for (int k = 0; k < q.m; k++)
       if (r[k].findex >= 0) r[k].findex += q.row0;
   }
   __syncthreads();
-  // --- rhs = c/h - J (v/h + inv(M) f_ext); cfm /= h (quickstep.cpp:832-857)
   for (int b = threadIdx.x; b < nb; b += blockDim.x) {
     int gb = c.W.b0 + b;
     float *t = bt + 32 * b;
@@ -1705,30 +1714,58 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
     t[20] = it.z + w.z * hinv;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < nrows; i += blockDim.x) {
-    Row &R = rows[i];
-    const float *t1 = bt + 32 * R.b1;
-    float s = 0.f;
-    for (int k = 0; k < 6; k++) s += R.J[k] * t1[15 + k];
-    float d = 0.f;
-    float im1 = B.invMass[c.W.b0 + R.b1];
-    for (int k = 0; k < 3; k++) R.iMJ[k] = im1 * R.J[k];
-    for (int k = 0; k < 3; k++) R.iMJ[3 + k] = t1[3 * k] * R.J[3] + t1[3 * k + 1] * R.J[4] + t1[3 * k + 2] * R.J[5];
-    for (int k = 0; k < 6; k++) d += R.iMJ[k] * R.J[k];
-    if (R.b2 >= 0) {
-      const float *t2 = bt + 32 * R.b2;
-      for (int k = 0; k < 6; k++) s += R.J[6 + k] * t2[15 + k];
-      float im2 = B.invMass[c.W.b0 + R.b2];
-      for (int k = 0; k < 3; k++) R.iMJ[6 + k] = im2 * R.J[6 + k];
-      for (int k = 0; k < 3; k++) R.iMJ[9 + k] = t2[3 * k] * R.J[9] + t2[3 * k + 1] * R.J[10] + t2[3 * k + 2] * R.J[11];
-      for (int k = 6; k < 12; k++) d += R.iMJ[k] * R.J[k];
-    } else {
-      for (int k = 6; k < 12; k++) R.iMJ[k] = 0.f;
+  for (int x = threadIdx.x; x < SOR_MAX_ROWS * nj; x += blockDim.x) {
+    const int i = nk + x / SOR_MAX_ROWS, k = x % SOR_MAX_ROWS;
+    if (k >= cons[i].m) continue;
+    Row *dst = rows + cons[i].row0 + k;
+    Row R = *dst;
+    finish_row(R, bt + 32 * R.b1, R.b2 >= 0 ? bt + 32 * R.b2 : nullptr, B.invMass[c.W.b0 + R.b1],
+               R.b2 >= 0 ? B.invMass[c.W.b0 + R.b2] : 0.f, hinv, P.sor_w);
+    store_row(dst, R);
+  }
+  for (int i = threadIdx.x; i < nk; i += blockDim.x) {
+    const Cons q = cons[i];
+    if (q.m <= 0) continue;
+    Row r[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      row_clear(r[k], P.cfm);
+      r[k].b1 = q.b1;
+      r[k].b2 = q.b2;
     }
-    R.rhs = R.rhs * hinv - s;
-    R.cfm = R.cfm * hinv;
-    R.ad = P.sor_w / (d + R.cfm);
-    R.lambda = 0.f;
+    const BodyPose s1 = load_pose(B, c.W.b0 + q.b1);
+    BodyPose s2;
+    if (q.b2 >= 0) s2 = load_pose(B, c.W.b0 + q.b2);
+    float3 cpos, cn;
+    float cd;
+    bool rev;
+    Surf s;
+    if (in.from_host) {
+      const ContactIn &ci = B.cin[B.cin_start[c.w] + q.src];
+      cpos = mk3(ci.pos[0], ci.pos[1], ci.pos[2]);
+      cn = mk3(ci.normal[0], ci.normal[1], ci.normal[2]);
+      cd = ci.depth;
+      rev = (ci.flags & JF_REVERSE) != 0;
+      s = host_surface(ci);
+    } else {
+      const ContactRec &cr = con[q.src];
+      cpos = mk3(cr.pos[0], cr.pos[1], cr.pos[2]);
+      cn = mk3(cr.normal[0], cr.normal[1], cr.normal[2]);
+      cd = cr.depth;
+      rev = (cr.flags & JF_REVERSE) != 0;
+      s = world_surface(P);
+    }
+    contact_info2(r, contact_info1(s), s, cpos, cn, cd, rev, s1, q.b2 >= 0 ? &s2 : nullptr, hinv,
+                  erp_of ? erp_of[i] : P.erp, P.min_depth, P.max_vel);
+    const float *t1 = bt + 32 * q.b1, *t2 = q.b2 >= 0 ? bt + 32 * q.b2 : nullptr;
+    const float im1 = B.invMass[c.W.b0 + q.b1], im2 = q.b2 >= 0 ? B.invMass[c.W.b0 + q.b2] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      if (k < q.m) {
+        if (r[k].findex >= 0) r[k].findex += q.row0;
+        finish_row(r[k], t1, t2, im1, im2, hinv, P.sor_w);
+        store_row(rows + q.row0 + k, r[k]);
+      }
   }
   __syncthreads();
   c.clk.lap(PH_ROWS);
