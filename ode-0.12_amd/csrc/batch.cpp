@@ -89,11 +89,15 @@ static int lds_share(const BatchImpl *b, int k) {
 }
 
 // The launch shape until one is set or tuned, by the number of worlds N, the
-// CUs and the worlds' size.  The kernel leaves a SIMD two wavefronts, a CU two
-// workgroups of 256, four of 128 or eight of 64.
+// CUs and the worlds' size.  The kernel leaves a SIMD two wavefronts, a CU one
+// workgroup of 512, two of 256, four of 128 or eight of 64.
 //  - N <= CUs: a CU each, and its whole LDS (a step of a pile of 1500 bodies
 //    in the reference order, whose ordering and forces then fit: 14.1 -> 5.7
-//    ms; two of 4096 bodies, coloured: 11.5 -> 11.0 ms).
+//    ms; two of 4096 bodies, coloured: 11.5 -> 11.0 ms).  512 lanes in the
+//    reference order, whose levels are built by all of them (5.5 -> 4.5 ms;
+//    128 exact solves 452 -> 409 us; a stack of 10 the same), and for large
+//    coloured worlds (4096 bodies: 10.2 -> 9.7 ms; at 1500 and below the idle
+//    half costs 3 % in barriers: 3.80 and 3.93 ms).
 //  - N <= 2 CUs: two on a CU, half its LDS each (600 worlds of 8 bodies take
 //    1.01 ms a pair of steps with 256 lanes and 0.77 with 128; 333 of 40
 //    bodies 1.49 and 1.61).
@@ -114,6 +118,7 @@ static void default_shape(BatchImpl *b) {
   for (const WorldInfo &w : b->wi) most = std::max(most, w.nb);
   b->wg = 256;
   if (!b->tol_on) {
+    if (N <= cu && (ref || mean >= 2048)) b->wg = 512;
     if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64)) b->wg = 64;
     else if (N > 2 * cu && (ref || most <= 128)) b->wg = 128;
   }

@@ -4,8 +4,8 @@
 // constraints whose (unique, hashed) priority is the largest among the still
 // uncoloured ones at both their bodies; they share no body.  First fit,
 // capped: the winners, in constraint order, each take the lowest colour that
-// neither body has taken and that has fewer than blockDim.x members (a colour
-// is then one pass of the block); past 64 colours, one colour of their own
+// neither body has taken and that has fewer than the workgroup's width (at
+// most 256) members (a colour is then one pass of the block); past 64 colours, one colour of their own
 // per round.
 //
 // Rounds work on lists that shrink (the constraints left, and the round's
@@ -49,7 +49,7 @@ __device__ __attribute__((noinline)) int colour_constraints(const Cons *cons, fl
   int *const bmax = PLACE == COL_IN_GLOBAL ? uniform_global(bmax_g) : (int *)(mask + nb);
   int *const col = PLACE == COL_IN_LDS ? bmax + nb : uniform_global(lists_g);
   int *const cb1 = col + ncons, *const cb2 = cb1 + ncons, *const left = cb2 + ncons, *const win = left + ncons;
-  const int nt = blockDim.x, t = threadIdx.x;
+  const int nt = blockDim.x, t = threadIdx.x, width = min(nt, COLOUR_WIDTH);
   auto taken = [&](int b) -> unsigned long long & {
     if constexpr (PLACE == COL_IN_GLOBAL) return *(unsigned long long *)(bt + 32 * b + 24);   // unused temp words
     else return mask[b];
@@ -143,7 +143,7 @@ __device__ __attribute__((noinline)) int colour_constraints(const Cons *cons, fl
       }
       __syncthreads();
       if (t < 64) {
-        const unsigned long long over = __ballot(sh.ccount[t] + sh.ccur[t] > nt);
+        const unsigned long long over = __ballot(sh.ccount[t] + sh.ccur[t] > width);
         if (t == 0) sh.ival[8] = over ? __ffsll((long long)over) - 1 : 64;
       }
       __syncthreads();
@@ -157,7 +157,7 @@ __device__ __attribute__((noinline)) int colour_constraints(const Cons *cons, fl
       }
       for (int k = t; k < cs; k += nt) sh.ccount[k] += sh.ccur[k];
       if (cs == 64) break;
-      const int room = nt - sh.ccount[cs];
+      const int room = width - sh.ccount[cs];
       int base = 0;
       for (int start = 0; start < nwin && base < room; start += nt) {
         const int x = start + t, i = x < nwin ? win[x] : 0;
@@ -169,7 +169,7 @@ __device__ __attribute__((noinline)) int colour_constraints(const Cons *cons, fl
       }
       __syncthreads();
       if (t == 0) {
-        sh.ccount[cs] = nt;
+        sh.ccount[cs] = width;
         if (cs < 32) sh.ival[9] |= (int)(1u << cs);
         else sh.ival[10] |= (int)(1u << (cs - 32));
       }

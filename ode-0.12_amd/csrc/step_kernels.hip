@@ -28,7 +28,8 @@
 
 namespace odemi {
 
-constexpr int WG = 256;
+constexpr int WG = 512;            // most lanes of a workgroup
+constexpr int COLOUR_WIDTH = 256;  // most constraints of a colour
 constexpr int MAX_COLORS_LDS = 256;   // colour buckets counted in LDS
 
 struct Shared {
