@@ -1,0 +1,111 @@
+"""Results do not depend on the launch shape, the placement of a working set in
+LDS or the way the state crosses to the host: the same bits on both sides of
+each line where one of them changes."""
+import numpy as np
+import pytest
+
+from conftest import say
+from odemi import scenes as sc
+
+pytestmark = pytest.mark.gpu
+
+
+def _pile(n, seed, spread=1.0):
+    """n spheres and boxes in a packed lattice, resting on a plane."""
+    rng = np.random.default_rng(seed)
+    b = sc._Builder()
+    b.geom(sc.PLANE, (0.0, 0.0, 1.0, 0.0))
+    side = max(1, int(np.ceil(n ** (1 / 3))))
+    for i in range(n):
+        x, y, z = i % side, (i // side) % side, i // side ** 2
+        p = (0.98 * spread * x, 0.98 * spread * y, 0.49 + 0.98 * z)
+        if rng.random() < 0.5:
+            b.sphere_body(p, 0.5, 1.0)
+        else:
+            b.box_body(p, (1.0, 1.0, 1.0), 1.0)
+    s = b.scene(dt=0.01, mu=0.5, seed=seed)
+    s.body_lvel = rng.normal(0, 0.1, (n, 3)).astype(np.float32).astype(np.float64)
+    return s
+
+
+@pytest.mark.parametrize("order", ["reference", "coloured"])
+@pytest.mark.parametrize("worlds", [1, 257, 513, 1025])
+def test_default_shape_gives_the_bits_of_256_lanes(odemi_mod, order, worlds):
+    """The default shape on both sides of one, two and four worlds per CU."""
+    o = odemi_mod.ORDER_REFERENCE if order == "reference" else odemi_mod.ORDER_COLORED
+    base = [_pile(n, n) for n in ((30,) if worlds == 1 else (1, 3, 9, 20, 27))]
+    ws = [base[w % len(base)] for w in range(worlds)]
+    out = []
+    for fixed in (False, True):
+        b = odemi_mod.Batch(ws, o)
+        if fixed:
+            b.set_launch_config(256, 1.0)
+        say("shape", order, worlds, b.launch_config()["wg"])
+        b.step(3)
+        out.append(b.state())
+        b.close()
+    assert np.array_equal(out[0], out[1])
+
+
+def test_wide_coloured_world(odemi_mod):
+    """512 lanes (the default of a large coloured world) and 256: colours stay
+    capped at 256, in every placement of the bodies' colouring state and of the
+    solver's (fixed sweeps)."""
+    s = _pile(2200, 5)
+    out = []
+    for lds in ("default", None, 60000, 20000, 0):
+        b = odemi_mod.Batch([s], odemi_mod.ORDER_COLORED)
+        if lds != "default":
+            b.set_launch_config(256, 1.0, lds)
+        say("wide", lds, b.launch_config()["wg"])
+        b.step(2)
+        out.append((b.state(), b.counters()["groups"]))
+        b.close()
+    for st, g in out[1:]:
+        assert g == out[0][1]
+        assert np.array_equal(st, out[0][0])
+
+
+@pytest.mark.parametrize("n", [1, 2, 12])
+def test_exact_lcp_placements_agree(odemi_mod, n):
+    """An island's workspace in LDS, all but its matrix, and in global memory."""
+    ws = [sc.box_stack(n, gap=-1e-3, seed=n), _pile(n, n, spread=1.5)]
+    out = []
+    for wg, lds in ((256, None), (64, 60000), (256, 30000), (128, 8192), (256, 0)):
+        say("exact", n, wg, lds)
+        b = odemi_mod.Batch(ws, odemi_mod.ORDER_REFERENCE)
+        b.set_launch_config(wg, 1.0, lds)
+        b.set_exact_lcp(15 * n + 15)
+        b.step(2)
+        assert b.counters()["overflow"] == 0
+        out.append(b.state())
+        b.close()
+    for st in out[1:]:
+        assert np.array_equal(st, out[0])
+
+
+@pytest.mark.parametrize("n", [1, 100, 20200])
+def test_state_crosses_unchanged(odemi_mod, n):
+    """set_state / state below and above the size that goes through pinned
+    memory (1 MB: 20 164 bodies), and a step from a state that was set."""
+    b1 = sc._Builder()
+    b1.geom(sc.PLANE, (0.0, 0.0, 1.0, 0.0))
+    per = min(n, 101)
+    for i in range(per):
+        b1.sphere_body((2.0 * i, 0.0, 1.0), 0.5, 1.0)
+    s = b1.scene(dt=0.01, mu=0.5, seed=1)
+    say("state", n)
+    a, b = (odemi_mod.Batch([s] * (n // per), odemi_mod.ORDER_COLORED) for _ in range(2))
+    st = a.state()
+    rng = np.random.default_rng(n)
+    q = rng.normal(0, 1, (len(st), 4))
+    st[:, 3:7] = q / np.linalg.norm(q, axis=1, keepdims=True)
+    st[:, 7:] = rng.normal(0, 1, (len(st), 6))
+    for x in (a, b):
+        x.set_state(st)
+        assert np.array_equal(x.state(), st)
+    a.step(2)
+    b.step(1)
+    b.set_state(b.state())
+    b.step(1)
+    assert np.array_equal(a.state(), b.state())
