@@ -62,9 +62,12 @@ struct dxWorld {
   bool device_newer = false;
   bool tape = false;
   DevBuf cin;                              // first contact (0) and count, 64 bytes on the contacts
-  // written by the kernels, read by the host without a copy
-  HostBuf collide_out;                     // counters, pairs, contact counts, contacts (dSpaceCollide)
-  HostBuf step_out;                        // what a step hands back (api_gather_kernel)
+  // counters, pairs, contact counts, contacts (dSpaceCollide), and what a step
+  // hands back (api_gather_kernel): up to XFER_PINNED bytes in pinned memory
+  // that the kernels write themselves, else in device memory (their small
+  // writes would cross the bus one by one)
+  HostBuf collide_out, step_out;
+  DevBuf collide_dev, step_dev;
   std::vector<float> stepped;              // the state of the last step, if the device's is the newer one
   DevBuf feedback, one_out, one_n;
   // the last dWorldQuickStep recorded for dWorldQuickStepBackward: pre-step
@@ -325,8 +328,14 @@ int build_mirror(dxWorld *w, dxSpace *sp) {
   w->mir_space = sp;
   w->pcap = wi.pcap;
   w->kcap = wi.kcap;
-  if (!w->collide_out.alloc(collide_out_contacts(wi.pcap) + sizeof(ContactRec) * wi.kcap) ||
-      !w->step_out.alloc(sizeof(int) * (CNT_N + 1 + w->mgeoms.size() + 13 * (size_t)w->mir->nb)) ||
+  const size_t cbytes = collide_out_contacts(wi.pcap) + sizeof(ContactRec) * wi.kcap;
+  const size_t sbytes = sizeof(int) * (CNT_N + 1 + w->mgeoms.size() + 13 * (size_t)w->mir->nb);
+  w->collide_out.release();
+  w->collide_dev.release();
+  w->step_out.release();
+  w->step_dev.release();
+  if (!(cbytes <= XFER_PINNED ? w->collide_out.alloc(cbytes) : w->collide_dev.alloc(cbytes)) ||
+      !(sbytes <= XFER_PINNED ? w->step_out.alloc(sbytes) : w->step_dev.alloc(sbytes)) ||
       !w->one_out.alloc(sizeof(CPoint) * MAX_SLOTS) || !w->one_n.alloc(16)) {
     report_error("device allocation failed");
     return 0;
@@ -662,9 +671,14 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
                                    m->stream));
   // counters, generator state, space order and state
   const size_t ng = w->mgeoms.size();
-  OD_HIP(launch_api_gather(D, m->nb, (int)ng, w->step_out.as<int>(), m->stream));
+  std::vector<int> big;
+  OD_HIP(launch_api_gather(D, m->nb, (int)ng, w->step_out.p ? w->step_out.as<int>() : w->step_dev.as<int>(), m->stream));
   OD_HIP(hipStreamSynchronize(m->stream));
-  const int *out = w->step_out.as<int>();
+  if (!w->step_out.p) {
+    big.resize(CNT_N + 1 + ng + 13 * (size_t)m->nb);
+    OD_HIP(hipMemcpy(big.data(), w->step_dev.p, sizeof(int) * big.size(), hipMemcpyDeviceToHost));
+  }
+  const int *out = w->step_out.p ? w->step_out.as<int>() : big.data();
   const int ovf = out[CNT_OVERFLOW];
   w->stepped.clear();
   if (ovf) {
@@ -1434,7 +1448,7 @@ void dSpaceCollide(dSpaceID s, void *data, dNearCallback *cb) {
   refresh_dev(m);
   DevBatch D = m->dev;
   const size_t o_counts = collide_out_counts(w->pcap), o_con = collide_out_contacts(w->pcap);
-  char *dout = w->collide_out.as<char>();
+  char *dout = w->collide_out.p ? w->collide_out.as<char>() : w->collide_dev.as<char>();
   D.counters = (int *)dout;
   D.pairs_out = (PairRec *)(dout + 64);
   D.pcount_out = (int *)(dout + o_counts);
@@ -1445,13 +1459,24 @@ void dSpaceCollide(dSpaceID s, void *data, dNearCallback *cb) {
     report_error("dSpaceCollide: collide kernel failed");
     return;
   }
-  const int *cnt = (const int *)dout;
+  // (copies: a callback may collide another space of the world)
+  const hipMemcpyKind kind = w->collide_out.p ? hipMemcpyHostToHost : hipMemcpyDeviceToHost;
+  auto fetch = [&](void *dst, size_t at, size_t bytes) {
+    if (kind == hipMemcpyHostToHost) std::memcpy(dst, dout + at, bytes);
+    else if (bytes) (void)hipMemcpy(dst, dout + at, bytes, kind);
+  };
+  int cnt[CNT_N];
+  fetch(cnt, 0, sizeof(cnt));
   if (cnt[CNT_OVERFLOW]) report_error("dSpaceCollide: device capacity exceeded (flags %d)", cnt[CNT_OVERFLOW]);
   const int np = cnt[CNT_PAIRS], nk = cnt[CNT_CONTACTS];
-  // (copies: a callback may collide another space of the world)
-  const std::vector<PairRec> pr((const PairRec *)(dout + 64), (const PairRec *)(dout + 64) + np);
-  const std::vector<int> pc((const int *)(dout + o_counts), (const int *)(dout + o_counts) + np);
-  const std::vector<ContactRec> cr((const ContactRec *)(dout + o_con), (const ContactRec *)(dout + o_con) + nk);
+  std::vector<PairRec> pr(np);
+  std::vector<int> pc(np);
+  std::vector<ContactRec> cr(nk);
+  if (np) {
+    fetch(pr.data(), 64, sizeof(PairRec) * np);
+    fetch(pc.data(), o_counts, sizeof(int) * np);
+  }
+  if (nk) fetch(cr.data(), o_con, sizeof(ContactRec) * nk);
   for (dxGeom *g : s->list) g->dirty = false;
   std::vector<dxGeom *> mg = w->mgeoms;
   int off = 0;
