@@ -296,6 +296,6 @@ __device__ void lcp_exact_world(const DevBatch &B, int w, Row *rows, float *bt, 
     else ok = lcp_exact_island<LCP_IN_GLOBAL>(rows, bt, ws, pool, r0, m, nb, sh);
     fail |= !ok;
   }
-  if (fail && t == 0) atomicOr(&B.counters[w * CNT_N + CNT_OVERFLOW], OVF_LCP);
+  if (fail && t == 0) raise_overflow(B, w, OVF_LCP);
   __syncthreads();
 }

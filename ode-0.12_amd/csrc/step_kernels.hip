@@ -63,6 +63,13 @@ struct PhaseClock {
   }
 };
 
+// Raises an overflow flag of world w; called by thread 0, the counters' only
+// writer.  Not an atomic OR: dSpaceCollide's counters are pinned host memory,
+// and the bus carries add, swap and compare-and-swap only.
+__device__ inline void raise_overflow(const DevBatch &B, int w, int flag) {
+  B.counters[w * CNT_N + CNT_OVERFLOW] |= flag;
+}
+
 // ------------------------------------------------------------------ block helpers
 
 __device__ inline int block_excl_scan(int v, int &total, Shared &sh) {
@@ -636,7 +643,7 @@ __device__ int phase_broadphase(const DevBatch &B, const Ctx &c, const WorldPara
     npairs += tot;
   }
   if (npairs > c.W.pcap) {
-    if (threadIdx.x == 0) atomicOr(&B.counters[c.w * CNT_N + CNT_OVERFLOW], OVF_PAIRS);
+    if (threadIdx.x == 0) raise_overflow(B, c.w, OVF_PAIRS);
     npairs = c.W.pcap;
   }
   {
@@ -736,7 +743,7 @@ __device__ int phase_narrowphase(const DevBatch &B, const Ctx &c, const WorldPar
     nk += tot;
   }
   if (nk > c.W.kcap) {
-    if (threadIdx.x == 0) atomicOr(&B.counters[c.w * CNT_N + CNT_OVERFLOW], OVF_CONTACTS);
+    if (threadIdx.x == 0) raise_overflow(B, c.w, OVF_CONTACTS);
     nk = c.W.kcap;
   }
   __syncthreads();
@@ -1651,7 +1658,7 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
     // not enough row storage: leave the world unchanged for this step (and
     // start the next solve from zero)
     if (threadIdx.x == 0) {
-      atomicOr(&B.counters[c.w * CNT_N + CNT_OVERFLOW], OVF_ROWS);
+      raise_overflow(B, c.w, OVF_ROWS);
       if (B.warm_n) B.warm_n[c.w] = -1;
       if (STAGE == 1) misc[MISC_SOR_READY] = 0;
     }
@@ -1914,7 +1921,7 @@ __device__ __attribute__((always_inline)) void phase_step(const DevBatch &B, con
   // a world whose state became non-finite is frozen (and reported) from now on
   if (threadIdx.x == 0 && sh.ival[13]) {
     P.dead = 1;
-    atomicOr(&B.counters[c.w * CNT_N + CNT_OVERFLOW], OVF_NONFINITE);
+    raise_overflow(B, c.w, OVF_NONFINITE);
   }
   c.clk.lap(PH_INTEGRATE);
 }
@@ -2021,7 +2028,7 @@ __device__ __attribute__((always_inline)) void run_world(const DevBatch &B, int 
     else in.nk = B.counters[w * CNT_N + CNT_CONTACTS];
     in.seq_base = 1 << 20;
     if (in.from_host && in.nk > c.W.kcap) {
-      if (threadIdx.x == 0) atomicOr(&B.counters[w * CNT_N + CNT_OVERFLOW], OVF_CONTACTS);
+      if (threadIdx.x == 0) raise_overflow(B, w, OVF_CONTACTS);
       in.nk = c.W.kcap;
     }
     phase_step<(MODE & MF_TOL) != 0, (MODE & MF_PRE) ? 1 : ((MODE & MF_POST) ? 2 : 0)>(B, c, P, in, sh, ref);
