@@ -1486,12 +1486,14 @@ void dSpaceCollide(dSpaceID s, void *data, dNearCallback *cb) {
     g_ctx.space = s;
     g_ctx.g1 = mg[pr[i].g1];
     g_ctx.g2 = mg[pr[i].g2];
+    // past the capacity (reported above) the counts exceed the contacts
+    const int n = std::min(pc[i], nk - off);
     g_ctx.con = cr.data() + off;
-    g_ctx.n = pc[i];
+    g_ctx.n = n;
     g_ctx.maxc = s->cached_maxc;
     cb(data, g_ctx.g1, g_ctx.g2);
     g_ctx = saved;
-    off += pc[i];
+    off += n;
   }
 }
 

@@ -3,6 +3,7 @@ what is handed out is what the device found room for, on both sides of the size
 up to which the results come back through pinned memory (1 MB)."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 from conftest import say
@@ -21,7 +22,7 @@ def _lib(odemi_mod):
             ("dInitODE2", I, [C.c_uint]), ("dWorldCreate", V, []), ("dWorldDestroy", None, [V]),
             ("dHashSpaceCreate", V, [V]), ("dSpaceDestroy", None, [V]), ("dBodyCreate", V, [V]),
             ("dBodySetPosition", None, [V, F, F, F]), ("dCreateBox", V, [V, F, F, F]), ("dGeomSetBody", None, [V, V]),
-            ("dSpaceCollide", None, [V, V, CB]), ("dSetErrorHandler", None, [V])]:
+            ("dSpaceCollide", None, [V, V, CB]), ("dCollide", I, [V, V, I, V, I]), ("dSetErrorHandler", None, [V])]:
         f = getattr(L, name)
         f.restype, f.argtypes = res, args
     return L
@@ -72,3 +73,29 @@ def test_overflow_is_reported(odemi_mod, overlapping, apart, pairs, flags):
     messages = _collide(_lib(odemi_mod), lambda _, a, b: seen.append((a, b)), overlapping, apart)
     assert len(seen) == pairs and len(set(seen)) == pairs
     assert messages == ([f"dSpaceCollide: device capacity exceeded (flags {flags})"] if flags else [])
+
+
+@pytest.mark.parametrize("overlapping,apart,contacts", [
+    (20, 0, 760),          # four a pair
+    (32, 0, 1984), (64, 0, 4096), (65, 0, 4096), (120, 1980, 12664),
+])
+def test_contacts_handed_out_are_the_devices(odemi_mod, overlapping, apart, contacts):
+    """dCollide in the callback gives contacts as far as there was room, and
+    none for the pairs after that."""
+    say("contacts", overlapping, apart)
+    L = _lib(odemi_mod)
+    rec = np.zeros((4, 32), np.float32)       # dContactGeom: pos 4, normal 4, depth, ...
+    counts, at = [], []
+
+    def near(_, g1, g2):
+        n = L.dCollide(g1, g2, 4, rec.ctypes.data, 128)
+        counts.append(n)
+        at.append(rec[:n, :9].copy())
+
+    _collide(L, near, overlapping, apart)
+    at = np.concatenate(at)
+    assert len(at) == sum(counts) == contacts
+    full = contacts // 4
+    assert counts[:full] == [4] * full and not any(counts[full:])
+    assert np.abs(at[:, :3]).max() < 0.6 and at[:, 8].min() > 0
+    assert np.allclose(np.linalg.norm(at[:, 4:7], axis=1), 1.0, atol=1e-5)
