@@ -476,6 +476,8 @@ ODE_API int dBatchAutotune(dBatchID b, int trial_steps);
 #define ODEMI_TUNE_FUSED_ONLY 2
 #define ODEMI_TUNE_NO_SOR_SPLIT 4   /* do not try the sweeps in a kernel of their own */
 ODE_API int dBatchAutotuneEx(dBatchID b, int trial_steps, int flags);
+/* The lanes of a workgroup (64, 128, 192, 256 or 512) and the broadphase's
+ * cell scale (1 to 8).  What the first call gives, the second takes. */
 ODE_API int dBatchGetLaunchConfig(dBatchID b, int *wg_size, float *cell_scale);
 ODE_API int dBatchSetLaunchConfig(dBatchID b, int wg_size, float cell_scale);
 /* LDS pool per workgroup in bytes (sort keys, colouring state and the

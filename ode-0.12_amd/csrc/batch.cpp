@@ -807,10 +807,10 @@ static int set_cell_scale(BatchImpl *b, float s) {
 }
 
 int batch_set_launch(BatchImpl *b, int wg, float cell_scale, int grid) {
-  if (wg != 64 && wg != 128 && wg != 192 && wg != 256) return 0;
+  if (wg != 64 && wg != 128 && wg != 192 && wg != 256 && wg != 512) return 0;
   if (!(cell_scale >= 1.0f && cell_scale <= 8.0f)) return 0;
   if (!b->shape_set) {
-    b->lds = lds_share(b, 2);   // the pool that goes with a shape set by hand
+    if (wg != b->wg) b->lds = lds_share(b, 2);   // the pool that goes with a width set by hand
     b->shape_set = true;
   }
   b->wg = wg;

@@ -109,3 +109,62 @@ def test_state_crosses_unchanged(odemi_mod, n):
     b.set_state(b.state())
     b.step(1)
     assert np.array_equal(a.state(), b.state())
+
+
+@pytest.mark.parametrize("order", ["reference", "coloured"])
+@pytest.mark.parametrize("worlds,bodies", [(1, 30), (1, 2200), (257, 9), (1025, 9)])
+def test_a_shape_that_is_read_can_be_set(odemi_mod, order, worlds, bodies):
+    """What launch_config() gives is accepted, with and without its pool and
+    grid, stays, and is the same shape."""
+    o = odemi_mod.ORDER_REFERENCE if order == "reference" else odemi_mod.ORDER_COLORED
+    ws = [_pile(bodies, 3)] * worlds
+    out = []
+    for again in (None, "all", "width"):
+        b = odemi_mod.Batch(ws, o)
+        c = b.launch_config()
+        say("read and set", order, worlds, bodies, again, c)
+        if again == "all":
+            b.set_launch_config(c["wg"], c["cell_scale"], c["lds"], grid=c["grid"])
+        elif again:
+            b.set_launch_config(c["wg"], c["cell_scale"])
+        assert b.launch_config() == c
+        b.step(1)
+        out.append(b.state())
+        b.close()
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
+@pytest.mark.parametrize("wg", [0, 32, 320, 384, 1024])
+def test_other_widths_are_refused(odemi_mod, wg):
+    b = odemi_mod.Batch([_pile(2, 1)], odemi_mod.ORDER_REFERENCE)
+    c = b.launch_config()
+    with pytest.raises(RuntimeError):
+        b.set_launch_config(wg, 1.0)
+    assert b.launch_config() == c
+
+
+def test_widest_workgroup_at_a_tolerance(odemi_mod):
+    """512 lanes set by hand while iterating to a tolerance, which takes 256 by
+    itself.  A bed of touching spheres (a pile of boxes has no single solution
+    and does not converge): forces within a few hundred times the residual of
+    1e-5 of the solution, so velocities within 1e-4 (dt = 0.01, mass 1)."""
+    b = sc._Builder()
+    b.geom(sc.PLANE, (0.0, 0.0, 1.0, 0.0))
+    for i in range(324):
+        b.sphere_body((0.998 * (i % 18), 0.998 * (i // 18), 0.499), 0.5, 1.0)
+    s = b.scene(dt=0.01, mu=0.5, seed=4)
+    s.body_lvel = np.random.default_rng(4).normal(0, 0.05, (324, 3)).astype(np.float32).astype(np.float64)
+    out = []
+    for wg in (256, 512):
+        b = odemi_mod.Batch([s], odemi_mod.ORDER_COLORED)
+        b.set_tolerance(1e-5, 20000, 10, accel=True)
+        assert b.launch_config()["wg"] == 256
+        b.set_launch_config(wg, 1.0, 65536)
+        say("tolerance", wg)
+        b.step(1)
+        unconverged, residual = b.solve_stats()
+        out.append(b.state())
+        say("residual", residual[0], "sweeps", b.world_counters()[0, 5], "differs", np.abs(out[0] - out[-1]).max())
+        assert unconverged[0] == 0 and residual[0] <= 1e-5
+        b.close()
+    assert np.abs(out[0] - out[1]).max() <= 1e-4
