@@ -869,9 +869,9 @@ int batch_phase_times(BatchImpl *b, double *ms) {
 }
 
 // Launch-shape search on the live batch (state saved and restored around
-// the trials): broadphase cell scale first, then workgroup size x LDS pool x
-// grid (one workgroup per world, or a persistent grid filling the CUs at the
-// kernel's occupancy for that shape).
+// the trials): the shape in use, with the broadphase cell scales, then
+// workgroup size x LDS pool x grid (one workgroup per world, or a persistent
+// grid filling the CUs at the kernel's occupancy for that shape).
 int batch_autotune(BatchImpl *b, int trial_steps, int flags) {
   if (trial_steps <= 0) trial_steps = 3;
   Snapshot snap;
@@ -885,39 +885,38 @@ int batch_autotune(BatchImpl *b, int trial_steps, int flags) {
   };
   double best = 1e30;
   b->sor_split = false;
-  if (!b->shape_set) batch_set_launch(b, 256, b->cell_scale, 0);
   int bw = b->wg, bg = b->grid, bl = b->lds;
   float bs = b->cell_scale;
-  const float scales[] = {1.0f, 1.5f, 2.0f};
+  auto consider = [&](int wg, float scale, int grid, int lds) {
+    double t;
+    if (!batch_set_launch(b, wg, scale, grid) || !batch_set_lds(b, lds) || !trial(t)) return;
+    // one launch per world (grid 0) must beat the persistent, size-ordered
+    // queue by 2 %: a single trial's noise is about that, and the queue's
+    // largest-first order is what bounds the tail of uneven batches
+    if (grid == 0) t *= 1.02;
+    if (t < best) { best = t; bw = wg; bs = scale; bg = grid; bl = lds; }
+  };
+  // the shape in use (the default's, unless one was set) is a candidate
+  const int wg0 = bw, lds0 = bl;
+  consider(bw, bs, bg, bl);
   if (!(flags & ODEMI_TUNE_KEEP_CELL))
-    for (float sc : scales) {
-      double t;
-      if (!batch_set_launch(b, bw, sc, 0) || !trial(t)) continue;
-      t *= 1.02;   // grid 0, as below
-      if (t < best) { best = t; bs = sc; bg = 0; }
-    }
-  const int wgs[] = {64, 128, 256};
+    for (float sc : {1.0f, 1.5f, 2.0f}) consider(wg0, sc, 0, lds0);
+  const int wgs[] = {64, 128, 256, 512};
   const int lds_div[] = {1, 2, 3, 4, 8};   // pool = LDS per CU / k
   int st = world_kernel_static_lds();
   // the fused kernel only: the two-kernel step (split) is switched off
   b->split = false;
   for (int wg : wgs)
     for (int k : lds_div) {
+      // 512 lanes fill a CU: for no more worlds than CUs, and the whole LDS
+      if (wg == 512 && (k > 1 || b->nworlds > b->cu_count)) continue;
       int lds = (b->lds_cu / k - st - 256) & ~255;
       if (lds < 0) lds = 0;
       if (lds > b->lds_max) lds = b->lds_max;
       int occ = world_kernel_occupancy(KM_FUSED, wg, lds);
       if (occ <= 0) continue;
       const int grids[] = {0, occ * b->cu_count};
-      for (int grid : grids) {
-        double t;
-        if (!batch_set_launch(b, wg, bs, grid) || !batch_set_lds(b, lds) || !trial(t)) continue;
-        // one launch per world (grid 0) must beat the persistent, size-ordered
-        // queue by 2 %: a single trial's noise is about that, and the queue's
-        // largest-first order is what bounds the tail of uneven batches
-        if (grid == 0) t *= 1.02;
-        if (t < best) { best = t; bw = wg; bg = grid; bl = lds; }
-      }
+      for (int grid : grids) consider(wg, bs, grid, lds);
     }
   batch_set_launch(b, bw, bs, bg);
   batch_set_lds(b, bl);
