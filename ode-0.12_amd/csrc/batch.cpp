@@ -110,7 +110,10 @@ static int lds_share(const BatchImpl *b, int k) {
 // lanes than 256 only where no world has more bodies than lanes, so that no
 // colour (its constraints share no body) reaches the cap.  Iterating to a
 // tolerance the block sums follow the width too, and it stays 256.
+// A width or a pool set by hand stays.  Narrow workgroups are for CUs shared
+// by many of them, so they don't go with a pool set by hand.
 static void default_shape(BatchImpl *b) {
+  if (b->wg_set) return;
   const int N = b->nworlds, cu = b->cu_count;
   const bool ref = b->order_mode == ORDER_REFERENCE;
   const double mean = (double)b->nb / N;
@@ -119,10 +122,12 @@ static void default_shape(BatchImpl *b) {
   b->wg = 256;
   if (!b->tol_on) {
     if (N <= cu && (ref || mean >= 2048)) b->wg = 512;
-    if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64)) b->wg = 64;
-    else if (N > 2 * cu && (ref || most <= 128)) b->wg = 128;
+    if (!b->lds_set) {
+      if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64)) b->wg = 64;
+      else if (N > 2 * cu && (ref || most <= 128)) b->wg = 128;
+    }
   }
-  b->lds = lds_share(b, N <= cu ? 1 : (b->wg == 256 ? 2 : (b->wg == 128 ? 4 : 8)));
+  if (!b->lds_set) b->lds = lds_share(b, N <= cu ? 1 : (b->wg == 256 ? 2 : (b->wg == 128 ? 4 : 8)));
 }
 
 template <class T>
@@ -783,7 +788,7 @@ int batch_set_tolerance(BatchImpl *b, float tol, int max_iterations, int check_e
       }))
     return 0;
   b->tol_on = tol > 0.f;
-  if (!b->shape_set) default_shape(b);
+  default_shape(b);
   destroy_graph(b);
   return 1;
 }
@@ -809,10 +814,8 @@ static int set_cell_scale(BatchImpl *b, float s) {
 int batch_set_launch(BatchImpl *b, int wg, float cell_scale, int grid) {
   if (wg != 64 && wg != 128 && wg != 192 && wg != 256 && wg != 512) return 0;
   if (!(cell_scale >= 1.0f && cell_scale <= 8.0f)) return 0;
-  if (!b->shape_set) {
-    if (wg != b->wg) b->lds = lds_share(b, 2);   // the pool that goes with a width set by hand
-    b->shape_set = true;
-  }
+  if (!b->wg_set && !b->lds_set && wg != b->wg) b->lds = lds_share(b, 2);   // what goes with a width set by hand
+  b->wg_set = true;
   b->wg = wg;
   b->grid = grid;
   if (!set_cell_scale(b, cell_scale)) return 0;
@@ -823,7 +826,8 @@ int batch_set_launch(BatchImpl *b, int wg, float cell_scale, int grid) {
 int batch_set_lds(BatchImpl *b, int bytes) {
   if (bytes < 0 || bytes > b->lds_max) return 0;
   b->lds = bytes & ~255;
-  b->shape_set = true;
+  b->lds_set = true;
+  default_shape(b);
   destroy_graph(b);
   return 1;
 }

@@ -76,7 +76,7 @@ struct BatchImpl {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int wg = 256;
-  bool shape_set = false; // wg or lds set by hand or tuned (else default_shape's)
+  bool wg_set = false, lds_set = false;   // set by hand or tuned (else default_shape's)
   int grid = 0;           // persistent grid size (0: one workgroup per world)
   float cell_scale = 1.0f;
   bool ctrl_set = false;

@@ -191,3 +191,25 @@ def test_tuning_is_not_slower_than_the_default(odemi_mod, keep_cell):
         say("tuned" if tuned else "default", b.launch_config(), ms[-1])
         b.close()
     assert ms[1] <= 1.1 * ms[0]
+
+
+@pytest.mark.parametrize("worlds", [1, 300, 600, 1100])
+def test_pool_and_tolerance_in_either_order(odemi_mod, worlds):
+    """A pool set by hand leaves the width to the solver mode, whichever is set
+    first: 256 lanes at a tolerance, and the same bits."""
+    base = [_pile(n, n) for n in (1, 9, 20, 27)]
+    ws = [base[w % len(base)] for w in range(worlds)]
+    out = []
+    for first in ("pool", "tolerance"):
+        b = odemi_mod.Batch(ws, odemi_mod.ORDER_COLORED)
+        for what in (first, "tolerance" if first == "pool" else "pool"):
+            if what == "pool":
+                b.L.dBatchSetLds(b.h, 40960)
+            else:
+                b.set_tolerance(1e-5, 400, 10, accel=True)
+        say("pool and tolerance", worlds, first, b.launch_config())
+        assert b.launch_config()["wg"] == 256 and b.launch_config()["lds"] == 40960
+        b.step(2)
+        out.append(b.state())
+        b.close()
+    assert np.array_equal(out[0], out[1])
