@@ -31,7 +31,8 @@ def _pile(n, seed, spread=1.0):
 @pytest.mark.parametrize("order", ["reference", "coloured"])
 @pytest.mark.parametrize("worlds", [1, 257, 513, 1025])
 def test_default_shape_gives_the_bits_of_256_lanes(odemi_mod, order, worlds):
-    """The default shape on both sides of one, two and four worlds per CU."""
+    """The default shape on both sides of one, two and four worlds per CU, by
+    the number of small worlds."""
     o = odemi_mod.ORDER_REFERENCE if order == "reference" else odemi_mod.ORDER_COLORED
     base = [_pile(n, n) for n in ((30,) if worlds == 1 else (1, 3, 9, 20, 27))]
     ws = [base[w % len(base)] for w in range(worlds)]
@@ -213,3 +214,35 @@ def test_pool_and_tolerance_in_either_order(odemi_mod, worlds):
         out.append(b.state())
         b.close()
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("bodies,worlds,wg", [(64, 1025, 64), (65, 1025, 128), (128, 513, 128), (129, 513, 256)])
+def test_narrow_workgroups_hold_a_whole_colour(odemi_mod, bodies, worlds, wg):
+    """Coloured order: the largest world at the width's bound, all its bodies
+    apart on a plane, so that one colour has a constraint of every body; the
+    bits and colours of 256 lanes."""
+    def spheres(n):
+        b = sc._Builder()
+        b.geom(sc.PLANE, (0.0, 0.0, 1.0, 0.0))
+        for i in range(n):
+            b.sphere_body((1.5 * (i % 12), 1.5 * (i // 12), 0.49), 0.5, 1.0)
+        s = b.scene(dt=0.01, mu=0.5, seed=n)
+        s.body_lvel = np.random.default_rng(n).normal(0, 0.2, (n, 3)).astype(np.float32).astype(np.float64)
+        s.body_lvel[:, 2] = 0
+        return s
+    ws = [spheres(bodies)] + [spheres(3)] * (worlds - 1)
+    out = []
+    for fixed in (False, True):
+        b = odemi_mod.Batch(ws, odemi_mod.ORDER_COLORED)
+        if fixed:
+            b.set_launch_config(256, 1.0)
+        else:
+            assert b.launch_config()["wg"] == wg
+        say("whole colour", bodies, worlds, b.launch_config()["wg"])
+        b.step(1)
+        wc = b.world_counters()
+        assert wc[0, 1] == bodies and wc[0, 3] == 1
+        b.step(2)
+        out.append((b.state(), wc[:, 3]))
+        b.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
