@@ -664,6 +664,7 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
     OD_HIP(hipMemcpyAsync(st + 2 * (size_t)m->nb, m->d.lvel.p, bytes, hipMemcpyDeviceToDevice, m->stream));
     OD_HIP(hipMemcpyAsync(st + 3 * (size_t)m->nb, m->d.avel.p, bytes, hipMemcpyDeviceToDevice, m->stream));
   }
+  w->stepped.clear();   // of the step before: from here on the device's state counts, also if this step fails late
   OD_HIP(launch_world_kernel(KM_API_STEP, D, 0, 1, 0, m->wg, 0, m->stream));
   if (record)
     OD_HIP(launch_api_tape_capture(D, dcin, nk, w->tape_con.as<adj::TapeContact<float>>(),
@@ -680,7 +681,6 @@ static int world_step_impl(dWorldID w, dReal stepsize, bool exact, const char *w
   }
   const int *out = w->step_out.p ? w->step_out.as<int>() : big.data();
   const int ovf = out[CNT_OVERFLOW];
-  w->stepped.clear();
   if (ovf) {
     report_error("%s: %s (flags %d)", who,
                  (ovf & OVF_LCP) ? "the LCP solve did not finish" : "device capacity exceeded", ovf);
