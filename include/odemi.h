@@ -549,8 +549,10 @@ ODE_API int dBatchTapeSetOptions(dBatchID b, int checkpoint_interval, float act_
  * recorded step's pre-state and contacts on the device (64 bytes per body
  * plus the contact capacity, per step), and dBatchStepBackward runs the
  * reverse sweep without replaying the checkpoint segments; the gradients
- * are the same bits.  No counterpart in the reference (which has no
- * adjoint). */
+ * are the same bits.  The kept steps and the buffers of dBatchStepBackward
+ * then stay allocated, also past dBatchTapeEnd, until on = 0 or the batch is
+ * destroyed; without kept steps each dBatchStepBackward frees its own.  No
+ * counterpart in the reference (which has no adjoint). */
 ODE_API int dBatchTapeKeepSteps(dBatchID b, int on);
 /* Totals of the last backward pass: adjoint-solve iterations, and contact
  * pairs whose dual-number collider disagreed with the tape (0 expected). */

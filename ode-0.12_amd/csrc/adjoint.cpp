@@ -124,8 +124,8 @@ int tape_keep_steps(BatchImpl *b, bool on) {
     t.kovf.release();
     t.kcon_off.release();
     t.kjnt.release();
-    for (DevBuf *d : {&t.back.seg_st, &t.back.seg_con, &t.back.seg_nk, &t.back.seg_jnt, &t.back.gbuf, &t.back.scr})
-      d->release();
+    for (DevBuf *d : {&t.back.con_off, &t.back.scr_off, &t.back.gbuf, &t.back.scr, &t.back.par, &t.back.stats}) d->release();
+    t.back.ncon = t.back.nscr = 0;
     if (t.kept) {
       t.kept = false;
       t.nsteps = 0;
@@ -195,7 +195,8 @@ int tape_backward(BatchImpl *b, int nsteps, const float *grad_out, float *grad_i
     return 0;
   }
   const int nb = b->nb, nw = b->nworlds, K = t.interval;
-  Tape::Back &k = t.back;
+  Tape::Back call;   // a replay's buffers go with the call
+  Tape::Back &k = t.kept ? t.back : call;
   if (!k.nscr) {
     // per-world offsets of contacts and adjoint scratch
     std::vector<long long> con_off(nw), scr_off(nw);

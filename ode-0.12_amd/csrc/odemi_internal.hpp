@@ -37,9 +37,11 @@ struct Tape {
   // the joint controls each recorded step ran with (replays re-apply them)
   DevBuf kctrl;
   std::vector<char> ctrl_on;
-  // the backward pass's buffers, kept from one call to the next
+  // the backward pass's buffers; with kept steps they stay from one call to
+  // the next, until tape_keep_steps(b, false)
   struct Back {
-    DevBuf con_off, scr_off, seg_st, seg_con, seg_nk, seg_jnt, gbuf, scr, par, stats, ctrl_save;
+    DevBuf con_off, scr_off, gbuf, scr, par, stats;
+    DevBuf seg_st, seg_con, seg_nk, seg_jnt, ctrl_save;   // of a replay, and the state after it
     Snapshot end;
     long long ncon = 0, nscr = 0;   // contacts and scratch floats of all worlds (con_off and scr_off set)
   } back;

@@ -466,3 +466,36 @@ def test_tape_refuses_joints_it_does_not_cover(odemi_mod):
             b.tape_begin(5)
     finally:
         b.close()
+
+
+def test_backward_gives_its_buffers_back(odemi_mod):
+    """Replaying, the backward pass's buffers go with the call; with kept steps
+    they stay with the kept ones until those are given up (2 MiB: the
+    granularity of the device's free memory)."""
+    import torch
+    say("adjoint: buffers")
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    for worlds in (2, 400):      # the first one loads the kernels
+        b = odemi_mod.Batch([contact_scene(7, 20, (0,))] * worlds, odemi_mod.ORDER_COLORED)
+        b.set_tolerance(1e-5, 400, 10)
+        b.tape_options(2)
+        b.step(1)
+        before = free()
+        for keep in (False, True, False):
+            b.tape_keep_steps(keep)
+            b.tape_begin(2)
+            b.step(2)
+            taped = free()
+            b.step_backward(2, np.ones((b.nb, 13), np.float32))
+            b.tape_end()
+            say("worlds", worlds, "keep", keep, "tape", before - taped, "and backward", before - free())
+            if worlds > 2 and not keep:
+                assert taped - free() < 2 << 20
+        b.tape_keep_steps(False)
+        if worlds > 2:
+            assert taped - free() < 2 << 20
+        b.close()
