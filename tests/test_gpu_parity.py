@@ -769,7 +769,7 @@ def test_autotune_keeps_state(odemi_mod):
     a.step(3)
     st = a.state()
     wg = a.autotune(1)
-    assert wg in (64, 128, 256)
+    assert wg in (64, 128, 256, 512)
     assert np.array_equal(a.state(), st)
     b = _batch(odemi_mod, ws)
     b.step(3)
