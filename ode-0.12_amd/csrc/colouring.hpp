@@ -5,8 +5,8 @@
 // uncoloured ones at both their bodies; they share no body.  First fit,
 // capped: the winners, in constraint order, each take the lowest colour that
 // neither body has taken and that has fewer than the workgroup's width (at
-// most 256) members (a colour is then one pass of the block); past 64 colours, one colour of their own
-// per round.
+// most 256) members (a colour is then one pass of the block); past 64 colours,
+// one colour of their own per round.
 //
 // Rounds work on lists that shrink (the constraints left, and the round's
 // winners, both in constraint order), not on all constraints again: a world

@@ -16,7 +16,7 @@
 // us for a stack of 10 boxes (120 rows), about 200 for a pile of 1500 bodies
 // (11 889 rows).  One lane per island in sequence, the kernel before this,
 // took 0.44 us (rows in LDS) to 1.3 us (in global memory) a row: the solve of
-// the stack went from 1.06 to 0.30 ms, that of the pile from 304 to 4.5 ms.
+// the stack went from 1.06 to 0.27 ms, that of the pile from 304 to 3.5 ms.
 //
 // Every 8 sweeps the order is shuffled; shuffle and levels are built by all
 // lanes as well:
@@ -52,7 +52,15 @@ enum { REF_NO_FRICTION = -1, REF_IDLE = -2 };
 // ahead of their level); everything in the world's scratch.
 enum { REF_IN_LDS = 0, REF_ROWS_GLOBAL = 1, REF_SCHED_GLOBAL = 2, REF_IN_GLOBAL = 3 };
 
-// worlds up to this many rows place their levels with one wavefront
+// Worlds up to this many rows place their levels with one wavefront, and relax
+// them with it where few levels are wider than it.  It saves the barriers of
+// worlds of few rows: against all wavefronts throughout, a pass of a stack of
+// 10 (120 rows) takes 370 for 395 us, of 24 (282 rows) 442 for 473, of a pile
+// of 30 bodies (186 rows) 616 for 664; 333 worlds of 360 rows, a world of 633
+// and worlds above the limit the same within 1 %; 333 worlds of 656 rows 1.66
+// for 1.60 ms (1.71 if they were relaxed by one wavefront whatever the levels'
+// width).  A limit of 256 rows costs the stack of 24 its gain, one of 4096
+// changes nothing beyond 2 %.
 constexpr int REF_SOLO_ROWS = 1024;
 
 // Bytes of the solve's working set: 6 fc floats per body and for no body
@@ -251,7 +259,8 @@ __device__ inline int ref_levels(const RefSched &W, const Row *R, int m, bool &s
       if (t == 0) { sh.lcount[0] = d; sh.lcount[1] = passes; }
     }
     __syncthreads();
-    // one wavefront relaxes the levels if few of them are wider than it
+    // one wavefront relaxes the levels if few of them are wider than it (up
+    // to a quarter more passes than levels; the limit above has both sides)
     d = sh.lcount[0];
     solo = sh.lcount[1] <= d + (d >> 2);
     __syncthreads();
