@@ -341,7 +341,7 @@ BatchImpl *batch_create_arrays(BatchArrays &A, int order_mode) {
   long long scratch = 0, warm = 0;
   for (auto &wi : A.wi) {
     wi.scratch = scratch;
-    scratch += scratch_layout(wi.nb, wi.ng, wi.nj, wi.pcap, wi.kcap, wi.rcap).total;
+    scratch += scratch_bytes(wi.nb, wi.ng, wi.nj, wi.pcap, wi.kcap, wi.rcap, b->order_mode == ORDER_REFERENCE);
     wi.warm = warm;
     warm += warm_bytes(wi.kcap, wi.nj);
   }

@@ -183,7 +183,7 @@ enum { PH_AABB = 0, PH_BROAD, PH_NARROW, PH_BODIES, PH_ROWS, PH_ORDER, PH_SOR, P
 
 struct ScratchLayout {
   long long aabb, gbig, gidx, glevel, gdb, cells, ecount, pairs, pkeys, pcount, contacts, cons, rows, btmp,
-      order, adjs, adj, island, color, misc, sor, total;
+      order, adjs, adj, island, color, misc, sor;
 };
 
 OD_HD inline long long od_align(long long x) { return (x + 255) & ~255LL; }
@@ -260,17 +260,20 @@ OD_HD inline ScratchLayout scratch_layout(int nb, int ng, int nj, int pcap, int 
   L.cons = o;     o = od_align(o + (long long)sizeof(Cons) * ncons);
   L.rows = o;     o = od_align(o + (long long)sizeof(Row) * rcap);
   L.btmp = o;     o = od_align(o + 4LL * 32 * nb);
-  L.order = o;    o = od_align(o + 4LL * (rcap + ncons + nb + 2LL * ng + 8));
+  L.order = o;    o = od_align(o + 4LL * (ncons + nb + 2LL * ng + 8));
   L.adjs = o;     o = od_align(o + 4LL * (nb + 1));
   L.adj = o;      o = od_align(o + 4LL * 2 * ncons);
   L.island = o;   o = od_align(o + 4LL * (6LL * nb + 2 * ncons + 3LL * ng + 16));
   L.color = o;    o = od_align(o + 4LL * (ncons + nb));
   L.misc = o;     o = od_align(o + 4LL * 64);
-  // the solver's working set: one of the two orders'
-  const long long sb = sor_bytes(nb, rcap, (int)ncons), rb = ref_bytes(nb, rcap);
-  L.sor = o;      o = od_align(o + (sb > rb ? sb : rb));
-  L.total = o;
+  L.sor = o;   // the solver's working set, last (scratch_bytes)
   return L;
+}
+
+// bytes of a world's scratch, with the solver's working set of the batch's order
+OD_HD inline long long scratch_bytes(int nb, int ng, int nj, int pcap, int kcap, int rcap, bool ref) {
+  const ScratchLayout L = scratch_layout(nb, ng, nj, pcap, kcap, rcap);
+  return od_align(L.sor + (ref ? ref_bytes(nb, rcap) : sor_bytes(nb, rcap, kcap + nj + 1)));
 }
 
 // All device pointers the kernels need.
