@@ -110,8 +110,8 @@ static int lds_share(const BatchImpl *b, int k) {
 // lanes than 256 only where no world has more bodies than lanes, so that no
 // colour (its constraints share no body) reaches the cap.  Iterating to a
 // tolerance the block sums follow the width too, and it stays 256.
-// A width or a pool set by hand stays.  Narrow workgroups are for CUs shared
-// by many of them, so they don't go with a pool set by hand.
+// A width or a pool set by hand stays; narrow workgroups go with a pool of
+// which a CU has room for as many.
 static void default_shape(BatchImpl *b) {
   if (b->wg_set) return;
   const int N = b->nworlds, cu = b->cu_count;
@@ -122,10 +122,9 @@ static void default_shape(BatchImpl *b) {
   b->wg = 256;
   if (!b->tol_on) {
     if (N <= cu && (ref || mean >= 2048)) b->wg = 512;
-    if (!b->lds_set) {
-      if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64)) b->wg = 64;
-      else if (N > 2 * cu && (ref || most <= 128)) b->wg = 128;
-    }
+    auto room = [&](int k) { return !b->lds_set || b->lds <= lds_share(b, k); };
+    if (N > 4 * cu && mean <= (ref ? 24 : 48) && (ref || most <= 64) && room(8)) b->wg = 64;
+    else if (N > 2 * cu && (ref || most <= 128) && room(4)) b->wg = 128;
   }
   if (!b->lds_set) b->lds = lds_share(b, N <= cu ? 1 : (b->wg == 256 ? 2 : (b->wg == 128 ? 4 : 8)));
 }

@@ -264,3 +264,26 @@ def test_scratch_is_the_batches_orders(odemi_mod):
         b.close()
     say("bytes", used)
     assert used[0] < used[1] - (48 << 20)
+
+
+@pytest.mark.parametrize("worlds,lds,wg", [(1, 1024, 512), (600, 4096, 128), (600, 49152, 256), (1100, 16384, 64),
+                                           (1100, 32768, 128), (1100, 65536, 256)])
+def test_width_that_goes_with_a_pool(odemi_mod, worlds, lds, wg):
+    """A pool set by hand takes the narrow workgroups of which a CU has room
+    for four (128 lanes) or eight (64); the bits are those of 256 lanes."""
+    base = [_pile(n, n) for n in (9, 20, 27)]
+    ws = [base[w % 3] for w in range(worlds)]
+    out = []
+    for fixed in (False, True):
+        b = odemi_mod.Batch(ws, odemi_mod.ORDER_REFERENCE)
+        if fixed:
+            b.set_launch_config(256, 1.0, lds)
+        else:
+            b.L.dBatchSetLds(b.h, lds)
+        c = b.launch_config()
+        say("width and pool", worlds, c)
+        assert (c["wg"], c["lds"]) == (256 if fixed else wg, lds)
+        b.step(2)
+        out.append(b.state())
+        b.close()
+    assert np.array_equal(out[0], out[1])
